@@ -192,109 +192,204 @@ __global__ __launch_bounds__(256) void bl4_encode_kernel(const float* __restrict
     }
 }
 
-// REF encoder (the reference's encode_blocklut_kernel,
-// vllm_lut/fast_encode.py:22-72): bf16 weights, one fp32[256] codebook,
-// blocks of block_size consecutive weights.  Per block: absmax = max |w|
-// (fp32, at least 1e-10); each weight w / absmax (IEEE fp32 division) gets
-// the index of the nearest codebook entry, the first one on equal distances
-// (a scan of all 256 entries: the codebook need not be sorted); absmax is
-// stored as bf16 (round to nearest even).  One wave per block; the codebook
-// sits in LDS and every lane reads the same entry (a broadcast).
-__global__ __launch_bounds__(256) void ref_encode_kernel(const uint16_t* __restrict__ w,
-                                                         const float* __restrict__ codebook, int64_t n,
-                                                         int block_size, int64_t nblocks,
-                                                         uint8_t* __restrict__ codes,
-                                                         uint16_t* __restrict__ absmax) {
-    __shared__ float s_cb[256];
-    s_cb[threadIdx.x] = codebook[threadIdx.x];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int64_t b = (int64_t)blockIdx.x * 4 + wv; b < nblocks; b += (int64_t)gridDim.x * 4) {
-        const int64_t start = b * block_size;
-        const int len = (int)min((int64_t)block_size, n - start);
-        float mx = 0.f;
-        for (int i = lane; i < len; i += 64) mx = fmaxf(mx, fabsf(bf16_to_f32(w[start + i])));
-        mx = fmaxf(wave_reduce_max(mx), 1e-10f);
-        for (int i = lane; i < len; i += 64) {
-            const float v = bf16_to_f32(w[start + i]) / mx;
-            float bd = fabsf(v - s_cb[0]);
-            int best = 0;
-#pragma unroll 8
-            for (int c = 1; c < 256; ++c) {
-                const float dd = fabsf(v - s_cb[c]);
-                if (dd < bd) {
-                    bd = dd;
-                    best = c;
-                }
-            }
-            codes[start + i] = (uint8_t)best;
-        }
-        if (lane == 0) absmax[b] = (uint16_t)f32_to_bf16(mx);
-    }
-}
-
-// The reference's two other REF encoding rules, one wave per block of
-// block_size weights, the codebook (or its midpoints) in LDS:
-//   kRule 0, LUTQuantizer.quantize (vllm_lut/quantizer.py:242-306, the
+// ---------------------------------------------------------------------------
+// REF encoders.  Three rules, one kernel:
+//   kEncode (the reference's encode_blocklut_kernel, vllm_lut/fast_encode.py:
+//     22-72): bf16 weights; absmax = max |w| of the block (fp32, at least
+//     1e-10); v = w / absmax (IEEE fp32 division); code = the nearest of 256
+//     codebook entries by |v - c| in fp32, the first one on equal distances
+//     (the codebook need not be sorted).
+//   kQuantizer, LUTQuantizer.quantize (vllm_lut/quantizer.py:242-306, the
 //     BLOCKLUT / NESTEDLUT branch; block_size = n is its global "LUT"
 //     branch): absmax = max |w| in the weights' dtype, at least 1e-10 in that
 //     dtype (:282-283); v = w / absmax, rounded to bf16 for bf16 weights (torch
-//     divides bf16 tensors in fp32 and rounds the result, :284); code = the
-//     first nearest of the ncb entries by |v - c| in fp32 (argmin, :293-296;
-//     the codebook need not be sorted).
-//   kRule 1, the offload runtime's encoder (runtime/model_offload.py:
+//     divides bf16 tensors in fp32 and rounds the result, :284); code as
+//     kEncode, among ncb entries (argmin, :293-296).
+//   kMidpoints, the offload runtime's encoder (runtime/model_offload.py:
 //     897-907): weights as fp32; absmax at least fp32(1e-12); v = w / absmax in
 //     fp32; code = the number of midpoints fl32(fl32(c_i + c_{i+1}) / 2) of the
 //     ascending codebook below v (np.searchsorted, side "left": a value on a
 //     midpoint takes the lower entry, NaN the last).
 // absmax is stored as bf16 (round to nearest even).
-template <int kRule, bool kBf16In>
-__global__ __launch_bounds__(256) void ref_quantize_kernel(const void* __restrict__ w, const float* __restrict__ cb,
-                                                           int ncb, int64_t n, int block_size, int64_t nblocks,
-                                                           uint8_t* __restrict__ codes,
-                                                           uint16_t* __restrict__ absmax) {
-    __shared__ float s_c[256];
+//
+// Comparing a weight with every entry costs 3 VALU ops per entry and weight
+// (2816 x 2048 weights, 256 entries: 142 us, 0.12 TB/s, VALU-bound).  Here a
+// CTA sorts the entries once (LDS) and a weight looks up, by its bucket of
+// 1024 over the entries' range, how many entries lie in lower buckets, then
+// steps to its neighbours in the sorted order: about 6 LDS reads and 45 VALU
+// ops a weight (18.4 us for the same weights).  The result is the scan's, bit for bit: rounding is
+// monotone, so the entries at the least rounded distance are a run of the
+// sorted order around v; the run is walked and its lowest index taken.  A run
+// (or an outlier-stretched bucket) only costs time.
+enum EncodeRule { kEncode = 0, kQuantizer = 1, kMidpoints = 2 };
+
+constexpr int kEncThreads = 512;
+constexpr int kEncBuckets = 1024;
+
+struct EncTable {
+    float v[258];                    // [0] NaN, then the non-NaN values ascending, then NaN
+    uint8_t idx[256];                // entry of each (equal values in entry order)
+    uint8_t first[kEncBuckets];      // sorted values in lower buckets
+    float lo, scale;
+    int n;                           // non-NaN values
+    float raw[256];
+};
+
+// Bucket of v: monotone in v (each step is, with NaN products taken as 0).
+__device__ __forceinline__ int enc_bucket(float v, float lo, float scale) {
+    return (int)fminf(fmaxf((v - lo) * scale, 0.f), (float)(kEncBuckets - 1));
+}
+
+// Sorts the m values of s.raw (every thread of the CTA calls it).
+__device__ void enc_build(EncTable& s, int m) {
     const int t = threadIdx.x;
-    if (kRule == 0 && t < ncb) s_c[t] = cb[t];
-    if (kRule == 1 && t + 1 < ncb) {
-        const float sum = cb[t] + cb[t + 1];
-        s_c[t] = sum * 0.5f;   // exact halving: equals numpy's fp32 sum / 2.0
+    const bool have = t < m && s.raw[t] == s.raw[t];
+    // ascending without NaN (as trained codebooks are): each value is in place
+    const int in_place = __syncthreads_and(t >= m || (have && (t == 0 || s.raw[t - 1] <= s.raw[t])));
+    const int n = __syncthreads_count(have);
+    if (t < 258) s.v[t] = __builtin_nanf("");
+    __syncthreads();
+    if (have) {
+        const float c = s.raw[t];
+        int r = t;
+        if (!in_place) {
+            r = 0;
+            for (int j = 0; j < m; ++j) {
+                const float u = s.raw[j];
+                r += (u < c) || (u == c && j < t);
+            }
+        }
+        s.v[r + 1] = c;
+        s.idx[r] = (uint8_t)t;
     }
     __syncthreads();
-    const int lane = t & 63, wv = t >> 6;
-    auto load = [&](int64_t i) __attribute__((always_inline)) {
-        return kBf16In ? bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[i]) : reinterpret_cast<const float*>(w)[i];
-    };
+    if (t == 0) {
+        const float lo = n ? s.v[1] : 0.f, d = n ? s.v[n] - lo : 0.f;
+        const bool ok = d > 0.f && d < INFINITY;   // (an infinite end: one bucket)
+        s.lo = ok ? lo : 0.f;
+        s.scale = ok ? (float)kEncBuckets / d : 0.f;
+        s.n = n;
+    }
+    __syncthreads();
+    for (int b = t; b < kEncBuckets; b += kEncThreads) {
+        int pos = 0;
+#pragma unroll
+        for (int step = 128; step >= 1; step >>= 1)
+            if (pos + step <= n && enc_bucket(s.v[pos + step], s.lo, s.scale) < b) pos += step;
+        s.first[b] = (uint8_t)pos;   // at most n - 1 for a bucket some v falls in
+    }
+    __syncthreads();
+}
+
+// Code of the normalised weight x.
+template <int kRule>
+__device__ __forceinline__ uint32_t enc_code(const EncTable& s, float x, float lo, float scale, int last, bool none) {
+    if (x != x) return kRule == kMidpoints ? (uint32_t)last : 0u;
+    int pos = s.first[enc_bucket(x, lo, scale)];
+    if constexpr (kRule == kMidpoints) {
+        while (s.v[pos + 1] < x) ++pos;
+        return (uint32_t)pos;
+    }
+    while (s.v[pos + 1] <= x) ++pos;
+    // neighbours: sorted value pos - 1 <= x < value pos (NaN: there is none)
+    const float dl = x - s.v[pos], du = s.v[pos + 1] - x;
+    const float d = fminf(dl, du);
+    if (none || !(d < INFINITY)) return 0u;   // the scan's start value stands
+    uint32_t best = 255u;
+    if (dl == d) {
+        int j = pos;
+        do best = min(best, (uint32_t)s.idx[--j]);
+        while (x - s.v[j] == d);
+    }
+    if (du == d) {
+        int j = pos;
+        do best = min(best, (uint32_t)s.idx[j++]);
+        while (s.v[j + 1] - x == d);
+    }
+    return best;
+}
+
+// kVec: blocks of 8 * 2^i <= 512 weights, 8 weights (16-byte loads) a lane;
+// else any block size, one wave per block.
+template <int kRule, bool kBf16In, bool kVec>
+__global__ __launch_bounds__(kEncThreads) void ref_encode_kernel(const void* __restrict__ w,
+                                                                 const float* __restrict__ cb, int ncb, int64_t n,
+                                                                 int block_size, int64_t nblocks,
+                                                                 uint8_t* __restrict__ codes,
+                                                                 uint16_t* __restrict__ absmax) {
+    __shared__ EncTable s;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    // values searched: the entries, or the midpoints between them
+    const int m = kRule == kMidpoints ? ncb - 1 : ncb;
+    if (t < m) s.raw[t] = kRule == kMidpoints ? (cb[t] + cb[t + 1]) * 0.5f : cb[t];   // (halving is exact)
+    __syncthreads();
+    enc_build(s, m);
+    const float lo = s.lo, scale = s.scale;
+    const bool none = kRule != kMidpoints && (s.n == 0 || s.raw[0] != s.raw[0]);   // entry 0 NaN: nothing is nearer
     // the clamp's bound in the dtype the reference clamps in
-    const float lo = kRule == 1 ? 1e-12f : kBf16In ? bf16_to_f32(f32_to_bf16(1e-10f)) : 1e-10f;
-    for (int64_t b = (int64_t)blockIdx.x * 4 + wv; b < nblocks; b += (int64_t)gridDim.x * 4) {
-        const int64_t start = b * block_size;
-        const int len = (int)min((int64_t)block_size, n - start);
-        float mx = 0.f;
-        for (int i = lane; i < len; i += 64) mx = fmaxf(mx, fabsf(load(start + i)));
-        mx = fmaxf(wave_reduce_max(mx), lo);
-        for (int i = lane; i < len; i += 64) {
-            float v = load(start + i) / mx;
-            int code;
-            if constexpr (kRule == 0) {
-                if (kBf16In) v = bf16_to_f32(f32_to_bf16(v));
-                float bd = fabsf(v - s_c[0]);
-                code = 0;
-                for (int c = 1; c < ncb; ++c) {
-                    const float dd = fabsf(v - s_c[c]);
-                    if (dd < bd) {
-                        bd = dd;
-                        code = c;
-                    }
+    const float floor_v = kRule == kMidpoints ? 1e-12f
+                          : kRule == kQuantizer && kBf16In ? bf16_to_f32(f32_to_bf16(1e-10f)) : 1e-10f;
+    auto code_of = [&](float wx, float mx) __attribute__((always_inline)) {
+        float x = wx / mx;
+        if (kRule == kQuantizer && kBf16In) x = bf16_to_f32(f32_to_bf16(x));
+        return enc_code<kRule>(s, x, lo, scale, ncb - 1, none);
+    };
+    if constexpr (kVec) {
+        const int lpb = block_size >> 3;   // lanes per block
+        for (int64_t i0 = ((int64_t)blockIdx.x * kEncThreads + t) * 8; i0 - 8 * lane < n;
+             i0 += (int64_t)gridDim.x * kEncThreads * 8) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = 0.f;
+            if (i0 + 8 <= n) {
+                if constexpr (kBf16In) {
+                    const u32x4_t v = *reinterpret_cast<const u32x4_t*>((const uint16_t*)w + i0);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = bf16_to_f32((v[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+                } else {
+                    const f32x4_t a = *reinterpret_cast<const f32x4_t*>((const float*)w + i0);
+                    const f32x4_t b = *reinterpret_cast<const f32x4_t*>((const float*)w + i0 + 4);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = j < 4 ? a[j] : b[j - 4];
                 }
             } else {
-                code = 0;
-                for (int c = 0; c + 1 < ncb; ++c) code += s_c[c] < v ? 1 : 0;
-                if (v != v) code = ncb - 1;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (i0 + j < n)
+                        x[j] = kBf16In ? bf16_to_f32(((const uint16_t*)w)[i0 + j]) : ((const float*)w)[i0 + j];
             }
-            codes[start + i] = (uint8_t)code;
+            float mx = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(x[j]));
+            for (int off = lpb >> 1; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+            mx = fmaxf(mx, floor_v);
+            uint32_t c[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c[j] = code_of(x[j], mx);
+            if (i0 + 8 <= n) {
+                *reinterpret_cast<u32x2_t*>(codes + i0) = u32x2_t{c[0] | c[1] << 8 | c[2] << 16 | c[3] << 24,
+                                                                  c[4] | c[5] << 8 | c[6] << 16 | c[7] << 24};
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (i0 + j < n) codes[i0 + j] = (uint8_t)c[j];
+            }
+            if ((lane & (lpb - 1)) == 0 && i0 < n) absmax[i0 / block_size] = (uint16_t)f32_to_bf16(mx);
         }
-        if (lane == 0) absmax[b] = (uint16_t)f32_to_bf16(mx);
+    } else {
+        auto load = [&](int64_t i) __attribute__((always_inline)) {
+            return kBf16In ? bf16_to_f32(reinterpret_cast<const uint16_t*>(w)[i]) : reinterpret_cast<const float*>(w)[i];
+        };
+        for (int64_t b = (int64_t)blockIdx.x * (kEncThreads / 64) + wv; b < nblocks;
+             b += (int64_t)gridDim.x * (kEncThreads / 64)) {
+            const int64_t start = b * block_size;
+            const int len = (int)min((int64_t)block_size, n - start);
+            float mx = 0.f;
+            for (int i = lane; i < len; i += 64) mx = fmaxf(mx, fabsf(load(start + i)));
+            mx = fmaxf(wave_reduce_max(mx), floor_v);
+            for (int i = lane; i < len; i += 64) codes[start + i] = (uint8_t)code_of(load(start + i), mx);
+            if (lane == 0) absmax[b] = (uint16_t)f32_to_bf16(mx);
+        }
     }
 }
 
@@ -379,35 +474,41 @@ int launch_kmeans_1d(const float* x, int64_t n, float* cent, int k, int n_iter, 
     return LUTMOE_OK;
 }
 
+// CTAs of the encoders: building the sorted table takes a CTA about as long
+// as 8 thousand weights, so the grid is no more than two CTAs of 8 waves per
+// CU, which loop.
+template <int kRule, bool kBf16In>
+static int ref_encode_launch(const void* w, const float* codebook, int ncb, int64_t n, int block_size, uint8_t* codes,
+                             uint16_t* absmax, hipStream_t s) {
+    const int64_t nblocks = (n + block_size - 1) / block_size;
+    // 8 weights a lane: whole lanes, a power of two of them per block, and
+    // aligned 16-byte (codes: 8-byte) accesses
+    const bool vec = block_size >= 8 && block_size <= 512 && (block_size & (block_size - 1)) == 0 &&
+                     (uintptr_t)w % 16 == 0 && (uintptr_t)codes % 8 == 0;
+    const int64_t per = kEncThreads * 8;
+    const int64_t want = vec ? (n + per - 1) / per : (nblocks + kEncThreads / 64 - 1) / (kEncThreads / 64);
+    const dim3 grid((unsigned)(want < 512 ? want : 512)), block(kEncThreads);
+    if (vec)
+        hipLaunchKernelGGL((ref_encode_kernel<kRule, kBf16In, true>), grid, block, 0, s, w, codebook, ncb, n,
+                           block_size, nblocks, codes, absmax);
+    else
+        hipLaunchKernelGGL((ref_encode_kernel<kRule, kBf16In, false>), grid, block, 0, s, w, codebook, ncb, n,
+                           block_size, nblocks, codes, absmax);
+    return check_launch();
+}
+
 int launch_ref_quantize(const void* w, bool bf16_in, const float* codebook, int ncb, int64_t n, int block_size,
                         int rule, uint8_t* codes, uint16_t* absmax, hipStream_t s) {
-    const int64_t nblocks = (n + block_size - 1) / block_size;
-    int64_t ctas = (nblocks + 3) / 4;
-    if (ctas > 65536) ctas = 65536;
-    const dim3 grid((unsigned)ctas), block(256);
-    if (rule == 0 && bf16_in)
-        hipLaunchKernelGGL((ref_quantize_kernel<0, true>), grid, block, 0, s, w, codebook, ncb, n, block_size, nblocks,
-                           codes, absmax);
-    else if (rule == 0)
-        hipLaunchKernelGGL((ref_quantize_kernel<0, false>), grid, block, 0, s, w, codebook, ncb, n, block_size,
-                           nblocks, codes, absmax);
-    else if (bf16_in)
-        hipLaunchKernelGGL((ref_quantize_kernel<1, true>), grid, block, 0, s, w, codebook, ncb, n, block_size, nblocks,
-                           codes, absmax);
-    else
-        hipLaunchKernelGGL((ref_quantize_kernel<1, false>), grid, block, 0, s, w, codebook, ncb, n, block_size,
-                           nblocks, codes, absmax);
-    return check_launch();
+    if (rule == LUTMOE_QRULE_QUANTIZER)
+        return bf16_in ? ref_encode_launch<kQuantizer, true>(w, codebook, ncb, n, block_size, codes, absmax, s)
+                       : ref_encode_launch<kQuantizer, false>(w, codebook, ncb, n, block_size, codes, absmax, s);
+    return bf16_in ? ref_encode_launch<kMidpoints, true>(w, codebook, ncb, n, block_size, codes, absmax, s)
+                   : ref_encode_launch<kMidpoints, false>(w, codebook, ncb, n, block_size, codes, absmax, s);
 }
 
 int launch_ref_encode(const uint16_t* w, const float* codebook, int64_t n, int block_size, uint8_t* codes,
                       uint16_t* absmax, hipStream_t s) {
-    const int64_t nblocks = (n + block_size - 1) / block_size;
-    int64_t ctas = (nblocks + 3) / 4;
-    if (ctas > 65536) ctas = 65536;
-    hipLaunchKernelGGL(ref_encode_kernel, dim3((unsigned)ctas), dim3(256), 0, s, w, codebook, n, block_size,
-                       nblocks, codes, absmax);
-    return check_launch();
+    return ref_encode_launch<kEncode, true>(w, codebook, 256, n, block_size, codes, absmax, s);
 }
 
 }  // namespace lutmoe_host

@@ -1021,6 +1021,54 @@ def test_ref_encode_bit_exact(gpu, n, block_size, sorted_cb):
     assert torch.equal(c2, codes.cpu()) and torch.equal(a2, am.cpu())
 
 
+def _encode_codebook(kind, rng):
+    cb = rng.uniform(-1, 1, 256).astype(np.float32)
+    if kind == "repeated":
+        cb = cb[rng.integers(0, 40, 256)]
+    elif kind == "close":          # spacing below the rounding of v - c: wide ties
+        cb = (np.float32(0.25) + np.arange(256, dtype=np.float32) * np.float32(2.0 ** -24))[rng.permutation(256)]
+    elif kind == "outlier":        # nearly every entry in one bucket of the range
+        cb = (cb * np.float32(1e-4)).astype(np.float32)
+        cb[[3, 200]] = [1e6, -1e6]
+    elif kind == "constant":
+        cb[:] = 0.5
+    elif kind == "special":        # signed zeros, infinities, NaN
+        cb[[0, 9, 17, 30, 31]] = [np.inf, -np.inf, np.nan, 0.0, -0.0]
+    elif kind == "first_nan":
+        cb[0] = np.nan
+    return cb
+
+
+@pytest.mark.parametrize("kind", ["repeated", "close", "outlier", "constant", "special", "first_nan"])
+@pytest.mark.parametrize("n,block_size,offset", [(8 * 4099, 8, 0), (512 * 9 + 13, 512, 0), (5000, 128, 3), (4100, 24, 0)])
+def test_ref_encode_equals_scan(gpu, kind, n, block_size, offset):
+    """The encoder's sorted search against the scan it stands for (the first entry at the
+    least fp32 distance; NaN distances never less) on codebooks where they could part:
+    equal entries, ties of rounded distances, one crowded bucket, infinities, NaN; smallest
+    and largest 8-a-lane blocks, short tails, a misaligned start, blocks off that path."""
+    import torch
+    from block_lut_amd import ops
+    rng = np.random.default_rng(n)
+    cb = _encode_codebook(kind, rng)
+    w = np.zeros(n + offset, np.float32)
+    w[offset:] = rng.standard_normal(n) * 0.02
+    w[offset + 5:offset + 40:7] = np.nan
+    wb = O.f32_to_bf16(w)
+    wt = torch.from_numpy(wb.view(np.int16)).view(torch.bfloat16).to(gpu)[offset:]
+    codes, am = ops.ref_encode(wt, torch.from_numpy(cb).to(gpu), block_size)
+    v = O.bf16_to_f32(wb[offset:])
+    nb = -(-n // block_size)
+    pad = np.pad(np.nan_to_num(np.abs(v)), (0, nb * block_size - n)).reshape(nb, block_size).max(1)
+    mx = np.maximum(pad, np.float32(1e-10)).astype(np.float32)
+    x = v / np.repeat(mx, block_size)[:n]
+    with np.errstate(invalid="ignore"):
+        d = np.abs(x[:, None] - cb[None, :])
+    d = np.where(np.isnan(d), np.inf, d)
+    ref = np.where(np.isnan(cb[0]) | np.isnan(x), 0, d.argmin(1)).astype(np.uint8)
+    assert np.array_equal(codes.cpu().numpy(), ref)
+    assert np.array_equal(am.view(torch.int16).cpu().numpy().view(np.uint16), O.f32_to_bf16(mx))
+
+
 def test_ref_quantize_rule_on_golden_vectors(gpu):
     """LUTQuantizer.quantize's rule on the GPU reproduces the vectors written from the
     reference itself (tests/golden/quantizer.npz: fp32 weights, a padded tail with an
