@@ -20,6 +20,7 @@
 // (vllm_lut/cuda_lut_gemv.py:23-80).
 #include "common.h"
 #include "kernels.h"
+#include "lut_core.h"
 
 using namespace lutmoe;
 
@@ -128,9 +129,8 @@ struct RefDec {
         }
     }
     __device__ __forceinline__ void stage(uint8_t*, int) const {}
-    // kDeq: the dequantised weight bf16(cb * absmax) times x (fused_lut_gemv,
-    // vllm_lut/fused_kernel.py:13-46); otherwise lut_gemv's (x * cb) * absmax
-    template <int TB, bool kDeq = false>
+    // lut_gemv's product order (x * cb) * absmax
+    template <int TB>
     __device__ __forceinline__ void dot(int r, const uint8_t*, int, const uint4 (&xq)[TB], int nt,
                                         float (&acc)[TB]) const {
         float s[TB];
@@ -139,8 +139,7 @@ struct RefDec {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint32_t word = j < 4 ? cw[r].x : cw[r].y;
-            const float cv = s_cb[(word >> (8 * (j & 3))) & 0xffu];
-            const float v = kDeq ? bf16_to_f32(f32_to_bf16(cv * am[r])) : cv;
+            const float v = s_cb[(word >> (8 * (j & 3))) & 0xffu];
 #pragma unroll
             for (int t = 0; t < TB; ++t) {
                 if (t < nt) {
@@ -152,7 +151,7 @@ struct RefDec {
             }
         }
 #pragma unroll
-        for (int t = 0; t < TB; ++t) acc[t] = kDeq ? acc[t] + s[t] : fmaf(s[t], am[r], acc[t]);
+        for (int t = 0; t < TB; ++t) acc[t] = fmaf(s[t], am[r], acc[t]);
     }
     // fp32 activations, lut_gemv's product order (x * cb) * absmax
     template <int TB>
@@ -293,102 +292,185 @@ __global__ __launch_bounds__(256) void gemv_kernel(lutmoe_weights w, int expert,
     }
 }
 
-// Reference-shaped single-vector GEMV on REF weights for any K / block size:
-// one wave per row, scalar lanes, exact reference product order
-// (x * cb) * absmax per element.  Used when the vector path's alignment
-// preconditions do not hold.
+// REF GEMV on the reference's raw tensors (lut_gemv, fused_lut_gemv).  A wave
+// owns R rows; lane l takes columns kC*l .. kC*l + kC-1 of every 64*kC-column
+// step, its codes, absmax and activations loaded for two steps before any is
+// used.  The fp32 codebook sits in the wave's own LDS (no barrier between the
+// waves).  kDeq: the dequantised weight bf16(cb * absmax) times x
+// (fused_lut_gemv, vllm_lut/fused_kernel.py:13-46); otherwise lut_gemv's
+// (x * cb) * absmax with the absmax factored out of a lane's columns.
+//
+// One matrix is a few MB, so what bounds it is the latency of one round of
+// loads and how many waves issue them: 2 rows a wave (1408 waves at 2816
+// rows) instead of 8: 2816 x 2048, one vector, 14.0 -> 4.1 us in a graph
+// (5.9 MB, 1.4 TB/s from the Infinity Cache; a launch alone is about 2).
+//
+// kAligned: K and block_size multiples of 16, 16-byte loads of 16 columns, one
+// absmax per lane and row step.  Else any K, block_size >= 8: 8 columns,
+// unaligned loads, at most one absmax block boundary inside them, the row's
+// last K % 8 columns element by element.
+struct RefRows {
+    const uint16_t* x;
+    const uint8_t* idx;
+    const uint16_t* cbh;    // bf16 codebook, or
+    const float* cbf;       // fp32 codebook
+    const uint16_t* absmax;
+    void* y;
+    int M, K, T, nb, bs, bs_shift, y_dtype;   // bs_shift: log2(bs), -1 if bs is no power of two
+};
+
+__device__ __forceinline__ uint32_t ref_block(const RefRows& a, uint32_t flat) {
+    return a.bs_shift >= 0 ? flat >> a.bs_shift : flat / (uint32_t)a.bs;
+}
+
+template <int R, int TB, bool kDeq, bool kAligned>
+__global__ __launch_bounds__(256) void ref_gemv_rows_kernel(RefRows a) {
+    constexpr int kC = kAligned ? 16 : 8;
+    constexpr int kStep = 64 * kC;
+    constexpr int kCW = kC / 4, kXW = kC / 2;   // code / activation dwords
+    __shared__ float s_cb[4][256];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int row0 = (blockIdx.x * 4 + wv) * R;
+    if (row0 >= a.M) return;
+    float cbv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        cbv[i] = a.cbf ? a.cbf[4 * lane + i] : bf16_to_f32(a.cbh[4 * lane + i]);
+    uint32_t flat0[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) flat0[r] = (uint32_t)min(row0 + r, a.M - 1) * (uint32_t)a.K;
+    const float* cb = s_cb[wv];
+    const int nwhole = a.K / kC;   // lane pieces of kC columns
+    const int nb1 = a.nb - 1;
+    for (int t0 = 0; t0 < a.T; t0 += TB) {
+        const int nt = min(TB, a.T - t0);
+        float acc[R][TB];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int t = 0; t < TB; ++t) acc[r][t] = 0.f;
+        for (int p0 = 0; p0 < nwhole; p0 += 128) {
+            uint32_t cw[2][R][kCW], xw[2][TB][kXW];
+            float am[2][R], am1[2][R];
+            int split[2][R];   // columns of the piece in the first absmax block
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                // past the row's last piece: that piece again, its sums dropped
+                const uint32_t c = (uint32_t)min(p0 + 64 * u + lane, nwhole - 1) * kC;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const uint32_t f = flat0[r] + c;
+                    __builtin_memcpy(cw[u][r], __builtin_assume_aligned(a.idx + f, kAligned ? 16 : 1), kC);
+                    const uint32_t b = ref_block(a, f);
+                    am[u][r] = bf16_to_f32(a.absmax[min((int)b, nb1)]);
+                    if constexpr (!kAligned) {
+                        split[u][r] = (int)min((b + 1) * (uint32_t)a.bs - f, 8u);
+                        am1[u][r] = bf16_to_f32(a.absmax[min((int)b + 1, nb1)]);
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < TB; ++t)
+                    __builtin_memcpy(xw[u][t], __builtin_assume_aligned(a.x + (int64_t)(t0 + min(t, nt - 1)) * a.K + c,
+                                                                        kAligned ? 16 : 2), 2 * kC);
+            }
+            if (p0 == 0 && t0 == 0) {
+                *reinterpret_cast<f32x4_t*>(&s_cb[wv][4 * lane]) = f32x4_t{cbv[0], cbv[1], cbv[2], cbv[3]};
+                wave_lds_sync();
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const bool ok = p0 + 64 * u + lane < nwhole;
+                float s[R][TB];
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) s[r][t] = 0.f;
+#pragma unroll
+                for (int j = 0; j < kC; ++j) {
+                    float xv[TB];
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) {
+                        const uint32_t xp = xw[u][t][j >> 1];
+                        xv[t] = (j & 1) ? __uint_as_float(xp & 0xffff0000u) : __uint_as_float(xp << 16);
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        float v = cb[(cw[u][r][j >> 2] >> (8 * (j & 3))) & 0xffu];
+                        if constexpr (!kAligned) v *= j < split[u][r] ? am[u][r] : am1[u][r];
+                        else if constexpr (kDeq) v *= am[u][r];
+                        if constexpr (kDeq) v = bf16_to_f32(f32_to_bf16(v));
+#pragma unroll
+                        for (int t = 0; t < TB; ++t) s[r][t] = fmaf(xv[t], v, s[r][t]);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) {
+                        const float v = kAligned && !kDeq ? fmaf(s[r][t], am[u][r], acc[r][t]) : acc[r][t] + s[r][t];
+                        acc[r][t] = ok ? v : acc[r][t];
+                    }
+            }
+        }
+        if constexpr (!kAligned) {
+            if (nwhole == 0 && t0 == 0) {
+                *reinterpret_cast<f32x4_t*>(&s_cb[wv][4 * lane]) = f32x4_t{cbv[0], cbv[1], cbv[2], cbv[3]};
+                wave_lds_sync();
+            }
+            const int c = nwhole * kC + lane;
+            if (c < a.K) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const uint32_t f = flat0[r] + (uint32_t)c;
+                    float v = cb[a.idx[f]] * bf16_to_f32(a.absmax[min((int)ref_block(a, f), nb1)]);
+                    if (kDeq) v = bf16_to_f32(f32_to_bf16(v));
+#pragma unroll
+                    for (int t = 0; t < TB; ++t)
+                        acc[r][t] = fmaf(bf16_to_f32(a.x[(int64_t)(t0 + min(t, nt - 1)) * a.K + c]), v, acc[r][t]);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            if (t >= nt) break;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float v = wave_reduce(acc[r][t]);
+                if (lane == r && row0 + r < a.M) {
+                    const int64_t o = (int64_t)(t0 + t) * a.M + row0 + r;
+                    if (a.y_dtype == LUTMOE_DTYPE_F32) ((float*)a.y)[o] = v;
+                    else ((uint16_t*)a.y)[o] = (uint16_t)f32_to_bf16(v);
+                }
+            }
+        }
+    }
+}
+
+// Absmax blocks of fewer than 8 elements: one wave per row, scalar lanes.
 template <bool kDeq>
-__global__ __launch_bounds__(256) void ref_gemv_generic_kernel(
-    const uint16_t* __restrict__ x, const uint8_t* __restrict__ idx, const uint16_t* __restrict__ cbh,
-    const float* __restrict__ cbf, const uint16_t* __restrict__ absmax, void* __restrict__ y, int M,
-    int K, int T, int nb, int bs, int y_dtype) {
+__global__ __launch_bounds__(256) void ref_gemv_generic_kernel(RefRows a) {
     __shared__ float s_cb[256];
-    for (int i = threadIdx.x; i < 256; i += 256) s_cb[i] = cbf ? cbf[i] : bf16_to_f32(cbh[i]);
+    s_cb[threadIdx.x] = a.cbf ? a.cbf[threadIdx.x] : bf16_to_f32(a.cbh[threadIdx.x]);
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= M) return;
-    for (int t = 0; t < T; ++t) {
+    if (row >= a.M) return;
+    for (int t = 0; t < a.T; ++t) {
         float acc = 0.f;
-        for (int c = lane; c < K; c += 64) {
-            const int64_t flat = (int64_t)row * K + c;
-            int64_t b = flat / bs;
-            b = b < nb ? b : nb - 1;
-            const float xv = bf16_to_f32(x[(int64_t)t * K + c]);
-            const float cv = s_cb[idx[flat]], av = bf16_to_f32(absmax[b]);
+        for (int c = lane; c < a.K; c += 64) {
+            const uint32_t flat = (uint32_t)row * (uint32_t)a.K + (uint32_t)c;
+            const float xv = bf16_to_f32(a.x[(int64_t)t * a.K + c]);
+            const float cv = s_cb[a.idx[flat]], av = bf16_to_f32(a.absmax[min((int)ref_block(a, flat), a.nb - 1)]);
             acc += kDeq ? xv * bf16_to_f32(f32_to_bf16(cv * av)) : xv * cv * av;
         }
-        acc = wave_sum(acc);
+        acc = wave_reduce(acc);
         if (lane == 0) {
-            const int64_t o = (int64_t)t * M + row;
-            if (y_dtype == LUTMOE_DTYPE_F32) ((float*)y)[o] = acc;
-            else ((uint16_t*)y)[o] = (uint16_t)f32_to_bf16(acc);
+            const int64_t o = (int64_t)t * a.M + row;
+            if (a.y_dtype == LUTMOE_DTYPE_F32) ((float*)a.y)[o] = acc;
+            else ((uint16_t*)a.y)[o] = (uint16_t)f32_to_bf16(acc);
         }
     }
 }
-
-// REF fast path through the octet machinery: wraps the raw reference tensors
-// in a one-expert weight description.
-template <int TB, bool kDeq>
-__global__ __launch_bounds__(256) void ref_gemv_fast_kernel(
-    const uint16_t* __restrict__ x, const uint8_t* __restrict__ idx, const uint16_t* __restrict__ cbh,
-    const float* __restrict__ cbf, const uint16_t* __restrict__ absmax, void* __restrict__ y, int M,
-    int K, int T, int nb, int bs, int y_dtype) {
-    __shared__ float s_cb[256];
-    for (int i = threadIdx.x; i < 256; i += 256) s_cb[i] = cbf ? cbf[i] : bf16_to_f32(cbh[i]);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int row0 = (blockIdx.x * 4 + wv) * kRows;
-    if (row0 >= M) return;
-    int rows[kRows];
-#pragma unroll
-    for (int r = 0; r < kRows; ++r) rows[r] = min(row0 + r, M - 1);
-    RefDec dec;
-    dec.codes = idx;
-    dec.absmax = absmax;
-    dec.s_cb = s_cb;
-    dec.K = K;
-    dec.nb = nb;
-    dec.bs = bs;
-    const int nch = (K + kChunk - 1) / kChunk;
-    for (int tb = 0; tb < T; tb += TB) {
-        const int nt = min(TB, T - tb);
-        const uint16_t* xrow[TB];
-#pragma unroll
-        for (int t = 0; t < TB; ++t) xrow[t] = x + (int64_t)(tb + min(t, nt - 1)) * K;
-        float acc[kRows][TB];
-#pragma unroll
-        for (int r = 0; r < kRows; ++r)
-#pragma unroll
-            for (int t = 0; t < TB; ++t) acc[r][t] = 0.f;
-        for (int c = 0; c < nch; ++c) {
-            // lane covers columns c*512 + 8*lane .. +7; valid when inside K
-            const bool ok = c * kChunk + 8 * lane < K;
-            uint4 xq[TB];
-#pragma unroll
-            for (int t = 0; t < TB; ++t)
-                xq[t] = (ok && t < nt) ? *reinterpret_cast<const uint4*>(xrow[t] + c * kChunk + 8 * lane)
-                                       : make_uint4(0u, 0u, 0u, 0u);
-            dec.load(rows, c, lane, ok);
-            if (ok) {
-#pragma unroll
-                for (int r = 0; r < kRows; ++r) dec.template dot<TB, kDeq>(r, nullptr, lane, xq, nt, acc[r]);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < kRows; ++r)
-#pragma unroll
-            for (int t = 0; t < TB; ++t) {
-                const float v = wave_sum(acc[r][t]);
-                if (lane == 0 && t < nt && row0 + r < M) {
-                    const int64_t o = (int64_t)(tb + t) * M + row0 + r;
-                    if (y_dtype == LUTMOE_DTYPE_F32) ((float*)y)[o] = v;
-                    else ((uint16_t*)y)[o] = (uint16_t)f32_to_bf16(v);
-                }
-            }
-    }
-}
-
 
 inline int tb_for(int T) { return T <= 1 ? 1 : T <= 2 ? 2 : 4; }
 
@@ -396,32 +478,31 @@ inline int tb_for(int T) { return T <= 1 ? 1 : T <= 2 ? 2 : 4; }
 
 namespace lutmoe_host {
 
+template <int R, bool kDeq, bool kAligned>
+static void ref_gemv_rows_launch(const RefRows& a, hipStream_t s) {
+    const dim3 grid((a.M + 4 * R - 1) / (4 * R)), block(256);
+    switch (tb_for(a.T)) {
+        case 1: hipLaunchKernelGGL((ref_gemv_rows_kernel<R, 1, kDeq, kAligned>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((ref_gemv_rows_kernel<R, 2, kDeq, kAligned>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((ref_gemv_rows_kernel<R, 4, kDeq, kAligned>), grid, block, 0, s, a); break;
+    }
+}
+
 template <bool kDeq>
-static int ref_gemv_dispatch(const uint16_t* x, const uint8_t* idx, const uint16_t* cb_bf16,
-                             const float* cb_f32, const uint16_t* absmax, void* y, int M, int K, int T,
-                             int num_blocks, int block_size, int y_dtype, hipStream_t s) {
-    const bool fast = (K % 8 == 0) && (block_size % 8 == 0) && ((uintptr_t)idx % 8 == 0) &&
-                      ((uintptr_t)x % 16 == 0);
-    if (!fast) {
-        hipLaunchKernelGGL(ref_gemv_generic_kernel<kDeq>, dim3((M + 3) / 4), dim3(256), 0, s, x, idx,
-                           cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype);
-        return check_launch();
-    }
-    const dim3 grid((M + 4 * kRows - 1) / (4 * kRows));
-    switch (tb_for(T)) {
-        case 1: hipLaunchKernelGGL((ref_gemv_fast_kernel<1, kDeq>), grid, dim3(256), 0, s, x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype); break;
-        case 2: hipLaunchKernelGGL((ref_gemv_fast_kernel<2, kDeq>), grid, dim3(256), 0, s, x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype); break;
-        default: hipLaunchKernelGGL((ref_gemv_fast_kernel<4, kDeq>), grid, dim3(256), 0, s, x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype); break;
-    }
+static int ref_gemv_dispatch(const RefRows& a, hipStream_t s) {
+    const bool aligned = a.K % 16 == 0 && a.bs % 16 == 0 && (uintptr_t)a.idx % 16 == 0 && (uintptr_t)a.x % 16 == 0;
+    if (aligned) ref_gemv_rows_launch<2, kDeq, true>(a, s);
+    else if (a.bs >= 8) ref_gemv_rows_launch<2, kDeq, false>(a, s);
+    else hipLaunchKernelGGL(ref_gemv_generic_kernel<kDeq>, dim3((a.M + 3) / 4), dim3(256), 0, s, a);
     return check_launch();
 }
 
 int launch_ref_gemv(const uint16_t* x, const uint8_t* idx, const uint16_t* cb_bf16,
                     const float* cb_f32, const uint16_t* absmax, void* y, int M, int K, int T,
                     int num_blocks, int block_size, int y_dtype, hipStream_t s, bool dequant) {
-    if (dequant)
-        return ref_gemv_dispatch<true>(x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype, s);
-    return ref_gemv_dispatch<false>(x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, y_dtype, s);
+    const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
+    const RefRows a{x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, shift, y_dtype};
+    return dequant ? ref_gemv_dispatch<true>(a, s) : ref_gemv_dispatch<false>(a, s);
 }
 
 template <class Dec, bool kXF32>

@@ -314,6 +314,34 @@ def test_ref_gemv_generic_path(gpu):
     assert rel_maxabs(y.cpu().numpy()[0], ref) <= TOL
 
 
+@pytest.mark.parametrize("M,K,bs,T", [(1, 16, 16, 1), (9, 2048, 128, 1), (7, 2064, 48, 3), (5, 33, 128, 2),
+                                      (6, 7, 8, 1), (8, 1001, 24, 5), (13, 520, 8, 4), (3, 1024 + 8, 128, 1),
+                                      (5, 96, 3, 2)])
+@pytest.mark.parametrize("deq", [False, True])
+def test_ref_gemv_shapes(gpu, M, K, bs, T, deq):
+    """The single-matrix REF GEMV at the edges of its paths: rows and 64-lane steps left over,
+    one step and one more, K that is no multiple of 16 or 8, absmax blocks that end inside a
+    lane's columns, blocks of fewer than 8; an absmax row one entry short (clamped)."""
+    import torch
+    from block_lut_amd import ops
+    rng = np.random.default_rng(M * K + T)
+    xb = _x(rng, T, K)
+    idx = rng.integers(0, 256, (M, K), dtype=np.uint8)
+    cb = golden_codebook()
+    nb = max(1, -(-M * K // bs) - 1)
+    am = O.f32_to_bf16((rng.random(nb) * 0.1 + 0.01).astype(np.float32))
+    y = ops.ref_gemv(to_dev_bf16(xb, gpu), torch.from_numpy(idx).to(gpu), to_dev_bf16(cb, gpu), to_dev_bf16(am, gpu),
+                     block_size=bs, out_dtype=torch.float32, dequantised=deq).cpu().numpy()
+    blk = np.minimum(np.arange(M * K) // bs, nb - 1)
+    w = O.bf16_to_f32(cb)[idx].astype(np.float64) * O.bf16_to_f32(am)[blk].reshape(M, K)
+    if deq:
+        w = O.bf16_to_f32(O.f32_to_bf16(w.astype(np.float32)))
+    # fp32 sums of K terms: at most K 2^-24 of the sum of magnitudes
+    x = O.bf16_to_f32(xb).astype(np.float64)
+    bound = (K + 4) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
+    assert (np.abs(y - x @ w.T) <= bound + 1e-30).all()
+
+
 def test_lut_gemv_reference_signature(gpu):
     """launch_lut_gemv_kernel: fp32 codebook, default stream, bf16 out."""
     import torch
