@@ -78,6 +78,7 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct MoeLayout {
     size_t route, topk_w, topk_ids, pair_ids, pair_w, offsets, perm, inv, active, sched, act, y, dact, dy, dw, total;
+    int dy_splits;   // K splits of the dense down projection that fit
 };
 
 // Room for two K-split partial results of the down projection when that is
@@ -104,9 +105,20 @@ MoeLayout moe_layout(const lutmoe_moe_desc* d, int T, int k) {
     // the dense shared expert: its activations, its weighted rows, token weights
     const size_t Is = d->dense_inter > 0 ? (size_t)d->dense_inter : 0;
     L.dact = o;     o = align_up(o + (Is ? (size_t)T * Is * 2 : 0));
-    L.dy = o;       o = align_up(o + (Is ? (size_t)T * d->hidden * 4 : 0));
     L.dw = o;       o = align_up(o + (Is ? (size_t)T * 4 : 0));
-    L.total = o;
+    // ... last, so that its K splits (up to 8, of up to 2048 rows in all) take
+    // what a workspace holds past one of them; a workspace that would pass the
+    // fixed scratch of lutmoe_moe_forward_noalloc only with them stays within
+    // it (so the size still grows with T)
+    L.dy = o;
+    const size_t row = (size_t)d->hidden * 4, one = (size_t)T * row;
+    size_t rows = (size_t)T * 8 < 2048 ? (size_t)T * 8 : 2048;
+    if (rows < (size_t)T) rows = T;
+    const size_t base = align_up(o + (Is ? one : 0));
+    size_t with = align_up(o + (Is ? rows * row : 0));
+    if (with > kNoallocScratch) with = kNoallocScratch;
+    L.total = base > with ? base : with;
+    L.dy_splits = one ? (int)((L.total - o) / one) : 1;
     return L;
 }
 
@@ -434,11 +446,12 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     const bool dense = d->dense_inter > 0;
     const float* addend = dense ? (const float*)(ws + L.dy) : nullptr;
     if (dense && (stages & LUTMOE_STAGE_GATE_UP) &&
-        (rc = launch_dense_gate_up(d, (const uint16_t*)x, T, !gemv, (uint16_t*)(ws + L.dact), (float*)(ws + L.dw), s)))
+        (rc = launch_dense_gate_up(d, (const uint16_t*)x, T, (uint16_t*)(ws + L.dact), (float*)(ws + L.dw), s)))
         return rc;
+    int naddend = 1;   // (the decode kernels add one array)
     if (dense && (stages & LUTMOE_STAGE_DOWN) &&
-        (rc = launch_dense_down(d, (const uint16_t*)(ws + L.dact), T, !gemv, (const float*)(ws + L.dw),
-                                (float*)(ws + L.dy), s)))
+        (rc = launch_dense_down(d, (const uint16_t*)(ws + L.dact), T, (const float*)(ws + L.dw),
+                                (float*)(ws + L.dy), gemv ? 1 : L.dy_splits, &naddend, s)))
         return rc;
     if (gemv) {
         // routing + permutation happen inside both decode kernels
@@ -482,7 +495,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
         if ((rc = launch_prefill_down(d, act, r, y, (int)P, (int)prefill_y_splits(P, d->hidden), &nsplit, s)))
             return rc;
         return launch_combine(y, r.inv, T, ke, d->hidden, out, out_dtype, s, nsplit, (int64_t)P * d->hidden,
-                              addend);
+                              addend, naddend);
     }
     return LUTMOE_OK;
 }

@@ -1392,7 +1392,7 @@ inline int persistent_ctas(int ncu, int64_t items) {
 namespace lutmoe_host {
 
 // Compute units of the current device (a per-device property cache).
-static int cu_count() {
+int cu_count() {
     static std::atomic<int> cache[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;

@@ -8,6 +8,9 @@
 
 namespace lutmoe_host {
 
+// noalloc.hip: the device scratch of lutmoe_moe_forward_noalloc, per GPU
+constexpr size_t kNoallocScratch = size_t(32) << 20;
+
 // dequant.hip
 int launch_ref_dequant(uint16_t* out, const uint8_t* idx, const uint16_t* absmax,
                        const uint16_t* cb, int64_t n_per_expert, int64_t nb_per_expert,
@@ -74,11 +77,15 @@ int launch_decode_v2(const lutmoe_moe_desc* d, const uint16_t* x, const float* t
 
 // dense.hip: a dense bf16 shared expert (d->dense_inter > 0).  gate_up:
 // tokw[t] = the shared weight of token t, act [T][Is] bf16; down: y [T][H]
-// fp32 = tokw[t] * (act[t] . W2s^T).  mfma: the MFMA tiles, else GEMVs.
-int launch_dense_gate_up(const lutmoe_moe_desc* d, const uint16_t* x, int T, bool mfma, uint16_t* act,
-                         float* tokw, hipStream_t s);
-int launch_dense_down(const lutmoe_moe_desc* d, const uint16_t* act, int T, bool mfma, const float* tokw, float* y,
-                      hipStream_t s);
+// fp32 = tokw[t] * (act[t] . W2s^T), as *nsplit <= max_split partial results
+// (K splits) T * H floats apart.
+int launch_dense_gate_up(const lutmoe_moe_desc* d, const uint16_t* x, int T, uint16_t* act, float* tokw,
+                         hipStream_t s);
+int launch_dense_down(const lutmoe_moe_desc* d, const uint16_t* act, int T, const float* tokw, float* y,
+                      int max_split, int* nsplit, hipStream_t s);
+
+// gemm.hip: compute units of the current device (0: unknown)
+int cu_count();
 
 // decode.hip: the one-token layer's weight loads alone (HBM floor measurement)
 size_t decode_stream_probe_ctas(const lutmoe_moe_desc* d, int ns, int which);
@@ -106,10 +113,11 @@ int launch_router_logits(const uint16_t* x, const uint16_t* gate, int T, int H, 
                          int round_bf16, hipStream_t s);
 // nsplit > 1: y_pos holds nsplit partial results (K splits of the down
 // projection), split_stride floats apart, summed per position first.
-// addend: NULL or fp32 [T][H] added to each token's sum before the rounding.
+// addend: NULL or naddend fp32 [T][H] arrays, one after another, added in
+// order to each token's sum before the rounding.
 int launch_combine(const float* y_pos, const int32_t* inv, int T, int k_eff, int H,
                    void* out, int out_dtype, hipStream_t s, int nsplit = 1, int64_t split_stride = 0,
-                   const float* addend = nullptr);
+                   const float* addend = nullptr, int naddend = 1);
 
 // gemm.hip (prefill, MFMA)
 int launch_prefill_gate_up(const lutmoe_moe_desc* d, const uint16_t* x, const MoeRouting& r,

@@ -23,7 +23,7 @@
 
 namespace {
 
-constexpr size_t kScratchBytes = size_t(32) << 20;   // 32 MiB per GPU
+constexpr size_t kScratchBytes = lutmoe_host::kNoallocScratch;   // 32 MiB per GPU
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];

@@ -365,8 +365,8 @@ __global__ __launch_bounds__(1024) void permute_chunk_kernel(PairSrc ps, int P, 
 
 // out[t] = sum over the token's positions p (slot order) of y[p], each y[p]
 // itself the sum of nsplit partial rows (K-split down projection) at stride
-// sstride, added in split order; plus addend[t] when given; one rounding to
-// the output dtype.  CTA (t, x) covers columns [1024x, 1024x + 1024) of token
+// sstride, added in split order; plus the naddend rows addend[a][t] when given (in
+// order); one rounding to the output dtype.  CTA (t, x) covers columns [1024x, 1024x + 1024) of token
 // t, 4 a thread: the token's positions are the same in the whole CTA (scalar
 // loads), and a thread issues the loads of all its positions' rows before it
 // adds them (in slot order, as one pass over the positions would).  The rows
@@ -376,7 +376,7 @@ constexpr int kCombineMaxKe = 16;   // k + shared experts (the entry points chec
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ y, const int32_t* __restrict__ inv,
                                                       int T, int ke, int H, void* __restrict__ out,
                                                       int out_dtype, int nsplit, int64_t sstride,
-                                                      const float* __restrict__ addend) {
+                                                      const float* __restrict__ addend, int naddend) {
     const int t = blockIdx.x;
     const int h = blockIdx.y * 1024 + threadIdx.x * 4;
     if (h >= H) return;
@@ -400,7 +400,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 #pragma unroll
     for (int q = 0; q < kCombineMaxKe; ++q)
         if (pos[q] >= 0) sum += v[q];
-    if (addend) sum += *reinterpret_cast<const f32x4_t*>(addend + (int64_t)t * H + h);
+    if (addend)
+        for (int a = 0; a < naddend; ++a)
+            sum += *reinterpret_cast<const f32x4_t*>(addend + ((int64_t)a * T + t) * H + h);
     if (out_dtype == LUTMOE_DTYPE_F32) {
         *reinterpret_cast<f32x4_t*>((float*)out + (int64_t)t * H + h) = sum;
     } else {
@@ -481,10 +483,10 @@ int launch_route_pairs(const int32_t* topk_ids, const float* topk_w, int T, int 
 
 int launch_combine(const float* y_pos, const int32_t* inv, int T, int k_eff, int H, void* out,
                    int out_dtype, hipStream_t s, int nsplit, int64_t split_stride,
-                   const float* addend) {
+                   const float* addend, int naddend) {
     if (k_eff > kCombineMaxKe) return LUTMOE_EUNSUPPORTED;
     hipLaunchKernelGGL(combine_kernel, dim3((unsigned)T, (unsigned)((H + 1023) / 1024)), dim3(256), 0, s, y_pos,
-                       inv, T, k_eff, H, out, out_dtype, nsplit, split_stride, addend);
+                       inv, T, k_eff, H, out, out_dtype, nsplit, split_stride, addend, naddend);
     return check_launch();
 }
 

@@ -1619,3 +1619,36 @@ def test_moe_layer_dense_shared_expert(gpu, T, path, gated, logits):
     # the dense expert moves the result well past the bar: dropping it fails
     ref_wo = O.moe_layer(xb, rids, rw, w13.deq_f32, w2.deq_f32, shared=shared[:S], shared_w=sw)
     assert rel_maxabs(ref_wo, ref) > 50 * TOL
+
+
+@pytest.mark.parametrize("T,H,Is", [(4, 128, 64), (5, 128, 64), (16, 192, 640), (17, 128, 576), (32, 64, 128),
+                                    (33, 192, 64), (64, 128, 2112), (65, 192, 2048), (129, 128, 1088),
+                                    (1024, 64, 1536), (1025, 192, 192)])
+def test_dense_shared_expert_shapes(gpu, T, H, Is):
+    """The dense shared expert's kernels at their edges (4 / 64 tokens, tiles of 64, 128 and
+    256 tokens and 128 weight rows, K steps left over by the waves or the ring's stages, the
+    down projection split over K), each result against float64 within its fp32 sums and the
+    bf16 rounding of the activations between the projections."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    E, k, I = 2, 1, 64
+    w13, w2 = _moe_case("bl4", E, 0, H, I, seed=9)
+    d13, d2, _, _ = dense_shared_weights(gpu, Is, H, T)
+    rng = np.random.default_rng(T + H)
+    gate = to_dev_bf16(O.f32_to_bf16((rng.standard_normal(H) * 0.05).astype(np.float32)), gpu)
+    x = to_dev_bf16(_x(rng, T, H), gpu)
+    ids = torch.full((T, k), -1, dtype=torch.int32, device=gpu)      # no routed expert
+    wts = torch.zeros((T, k), device=gpu)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 0, dense_shared=(d13, d2), shared_gate=gate)
+    out = ops.moe_forward(moe, x, wts, ids, out_dtype=torch.float32, path=ops.PATH_MFMA).double()
+    xd = x.double()
+    h = xd @ d13.double().T
+    act = torch.nn.functional.silu(h[:, :Is]) * h[:, Is:]
+    w = torch.sigmoid(xd @ gate.double())[:, None]
+    ref = (act.to(torch.bfloat16).double() @ d2.double().T) * w
+    # an activation on a bf16 rounding boundary may round to the neighbour (2^-8 of it); the
+    # fp32 sums of both projections and the sigmoid add about 1e-5
+    bound = ((act.abs() * 2.0 ** -8).pow(2) @ d2.double().pow(2).T).sqrt() * w * 4 + 1e-5 * ref.abs().max()
+    assert ((out - ref).abs() <= bound).all()
+    assert ((out - ref).norm() / ref.norm()) < 1e-3
