@@ -27,6 +27,10 @@ FMT_NESTED = 2
 QRULE_QUANTIZER = 0
 QRULE_MIDPOINTS = 1
 
+ROUTE_RENORM = 1
+ROUTE_BF16_WEIGHTS = 2
+ROUTE_BF16_LOGITS = 4
+
 STAGE_ROUTE = 1
 STAGE_GATE_UP = 2
 STAGE_DOWN = 4
@@ -117,6 +121,7 @@ PROTOTYPES = {
     "lutmoe_moe_forward": (I32, [DP, P, P, P, I32, I32, P, I32, P, SZ, I32, P]),
     "lutmoe_moe_forward_stages": (I32, [DP, P, P, P, I32, I32, P, I32, P, SZ, I32, I32, P]),
     "lutmoe_moe_forward_logits": (I32, [DP, P, P, I32, I32, I32, F32, P, I32, P, SZ, I32, I32, P]),
+    "lutmoe_moe_forward_logits_ex": (I32, [DP, P, P, I32, I32, I32, F32, P, I32, P, SZ, I32, I32, P]),
     "lutmoe_moe_forward_noalloc": (I32, [DP, P, P, P, I32, I32, P, I32, I32, P]),
     "lutmoe_noalloc_prepare": (I32, []),
     "lutmoe_bl4_encode": (I32, [P, I64, I32, P, P, P]),

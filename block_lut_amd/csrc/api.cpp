@@ -357,7 +357,7 @@ int lutmoe_route_topk(const float* logits, int T, int E, int k, int renormalize,
     if (E > 4096) return LUTMOE_EUNSUPPORTED;
     if (T == 0) return LUTMOE_OK;
     if (!logits || !topk_w || !topk_ids) return LUTMOE_EINVAL;
-    return launch_route_topk(logits, T, E, k, renormalize, scaling, topk_w, topk_ids,
+    return launch_route_topk(logits, false, T, E, k, renormalize ? 1 : 0, scaling, topk_w, topk_ids,
                              stream_of(stream));
 }
 
@@ -408,7 +408,7 @@ namespace lutmoe_host {
 // Shared body of the MoE entry points.  Exactly one of (topk_w, topk_ids) and
 // logits is given.
 int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_w,
-                     const int32_t* topk_ids, const float* logits, int T, int k, int renorm,
+                     const int32_t* topk_ids, const void* logits, int T, int k, int flags,
                      float scaling, void* out, int out_dtype, void* workspace, size_t ws_bytes,
                      int force_path, int stages, void* stream) {
     if (stages <= 0 || stages > LUTMOE_STAGE_ALL) return LUTMOE_EINVAL;
@@ -421,6 +421,9 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     const bool by_logits = logits != nullptr;
     if (!x || !out || !workspace || (!by_logits && (!topk_w || !topk_ids))) return LUTMOE_EINVAL;
     if (by_logits && d->num_routed > 320) return LUTMOE_EUNSUPPORTED;
+    const int renorm = flags & (LUTMOE_ROUTE_RENORM | LUTMOE_ROUTE_BF16_WEIGHTS);
+    const bool logits_bf16 = (flags & LUTMOE_ROUTE_BF16_LOGITS) != 0;
+    if (logits_bf16 && T <= 64) return LUTMOE_EUNSUPPORTED;
     if (!aligned(x, 16) || !aligned(out, 16) || !aligned(workspace, 256)) return LUTMOE_EALIGN;
     const MoeLayout L = moe_layout(d, T, k);
     if (ws_bytes < L.total) return LUTMOE_EWORKSPACE;
@@ -429,6 +432,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     if (P >= (1ll << 31) / (d->hidden > d->inter ? d->hidden : d->inter)) return LUTMOE_EUNSUPPORTED;
     const bool lds_ok = P * 8 * 4 <= 48 * 1024;
     bool gemv = force_path == 1 || (force_path == 0 && T <= 32 && lds_ok);
+    if (gemv && logits_bf16) return LUTMOE_EUNSUPPORTED;
     if (gemv && !lds_ok) return LUTMOE_EUNSUPPORTED;
     // the decode-layer kernels take up to 320 experts and 512 (token, slot)
     // pairs; anything else runs on the grouped MFMA path
@@ -455,7 +459,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
         return rc;
     if (gemv) {
         // routing + permutation happen inside both decode kernels
-        return launch_decode_v2(d, (const uint16_t*)x, topk_w, topk_ids, logits, T, k, renorm,
+        return launch_decode_v2(d, (const uint16_t*)x, topk_w, topk_ids, (const float*)logits, T, k, renorm,
                                 scaling, act, ws + L.route, (float*)(ws + L.y), out, out_dtype, stages, s, addend);
     }
     int32_t* pair_ids = (int32_t*)(ws + L.pair_ids);
@@ -475,7 +479,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
         if (by_logits) {
             float* tw = (float*)(ws + L.topk_w);
             int32_t* ti = (int32_t*)(ws + L.topk_ids);
-            if ((rc = launch_route_topk(logits, T, E, k, renorm, scaling, tw, ti, s))) return rc;
+            if ((rc = launch_route_topk(logits, logits_bf16, T, E, k, renorm, scaling, tw, ti, s))) return rc;
             topk_w = tw;
             topk_ids = ti;
         }
@@ -528,8 +532,17 @@ int lutmoe_moe_forward_logits(const lutmoe_moe_desc* d, const void* x, const flo
                               int out_dtype, void* workspace, size_t ws_bytes, int force_path,
                               int stages, void* stream) {
     if (!logits) return T == 0 ? LUTMOE_OK : LUTMOE_EINVAL;
-    return moe_forward_impl(d, x, nullptr, nullptr, logits, T, k, renormalize, scaling, out,
+    return moe_forward_impl(d, x, nullptr, nullptr, logits, T, k, renormalize ? LUTMOE_ROUTE_RENORM : 0, scaling, out,
                             out_dtype, workspace, ws_bytes, force_path, stages, stream);
+}
+
+int lutmoe_moe_forward_logits_ex(const lutmoe_moe_desc* d, const void* x, const void* logits, int T, int k, int flags,
+                                 float scaling, void* out, int out_dtype, void* workspace, size_t ws_bytes,
+                                 int force_path, int stages, void* stream) {
+    if (flags & ~(LUTMOE_ROUTE_RENORM | LUTMOE_ROUTE_BF16_WEIGHTS | LUTMOE_ROUTE_BF16_LOGITS)) return LUTMOE_EINVAL;
+    if (!logits) return T == 0 ? LUTMOE_OK : LUTMOE_EINVAL;
+    return moe_forward_impl(d, x, nullptr, nullptr, logits, T, k, flags, scaling, out, out_dtype, workspace, ws_bytes,
+                            force_path, stages, stream);
 }
 
 // --------------------------------------------------------------- encoders

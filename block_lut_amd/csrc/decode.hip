@@ -98,7 +98,7 @@ struct DecodeArgs {
     const float* topk_w;       // [T][k] (ids mode)
     const int32_t* topk_ids;   // [T][k] (ids mode)
     const float* logits;       // [T][E] fp32 (logits mode: topk_ids == nullptr)
-    int T, k, renorm;
+    int T, k, renorm;          // renorm: kRenorm | kWeightsBf16
     int tb;                    // tokens per pass of the expert loops (1, 2 or 4)
     float scaling;
     uint16_t* act;             // [P][I] bf16
@@ -182,7 +182,7 @@ __device__ void cta_route(const DecodeArgs& A, RouteOut& R, RouteScratch& X) {
                 wave_lds_sync();
                 if (lane < k) {
                     const float pj = R.pw[t * ke + lane];
-                    R.pw[t * ke + lane] = (A.renorm ? pj / wsum : pj) * A.scaling;
+                    R.pw[t * ke + lane] = routed_weight(pj, wsum, A.renorm, A.scaling);
                 }
             } else {
                 float lsum = 0.f;
@@ -205,7 +205,7 @@ __device__ void cta_route(const DecodeArgs& A, RouteOut& R, RouteScratch& X) {
                 wave_lds_sync();
                 if (lane < k) {
                     const float pj = R.pw[t * ke + lane];
-                    R.pw[t * ke + lane] = (A.renorm ? pj / wsum : pj) * A.scaling;
+                    R.pw[t * ke + lane] = routed_weight(pj, wsum, A.renorm, A.scaling);
                 }
             }
             const float sw = A.d.shared_gate && S > 0
@@ -354,7 +354,7 @@ __device__ __forceinline__ WaveRoute wave_pairs(const DecodeArgs& A) {
                 }
                 if (lane == sel) key = INT_MIN;
             }
-            if (kWeights && lane >= t * ke && lane < t * ke + k) w = (A.renorm ? w / wsum : w) * A.scaling;
+            if (kWeights && lane >= t * ke && lane < t * ke + k) w = routed_weight(w, wsum, A.renorm, A.scaling);
             if (lane >= t * ke + k && lane < (t + 1) * ke) { e = E + lane - t * ke - k; w = 1.0f; }
         }
     }

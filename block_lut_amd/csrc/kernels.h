@@ -58,10 +58,11 @@ struct MoeRouting {
 };
 
 // api.cpp: the body shared by the MoE layer entry points (arguments as
-// lutmoe_moe_forward_stages, logits instead of topk_w/topk_ids when given),
+// lutmoe_moe_forward_stages, logits instead of topk_w/topk_ids when given, with
+// flags = the bits of lutmoe_moe_forward_logits_ex),
 // and the calling thread's lutmoe_last_error text.
 int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_w,
-                     const int32_t* topk_ids, const float* logits, int T, int k, int renorm,
+                     const int32_t* topk_ids, const void* logits, int T, int k, int flags,
                      float scaling, void* out, int out_dtype, void* workspace, size_t ws_bytes,
                      int force_path, int stages, void* stream);
 void set_last_error_text(const char* text);
@@ -93,7 +94,8 @@ int launch_decode_stream_probe(const lutmoe_moe_desc* d, const int32_t* ids, int
                                hipStream_t s);
 
 // route.hip
-int launch_route_topk(const float* logits, int T, int E, int k, int renorm, float scaling,
+// renorm: kRenorm | kWeightsBf16 (lut_core.h)
+int launch_route_topk(const void* logits, bool logits_bf16, int T, int E, int k, int renorm, float scaling,
                       float* w, int32_t* ids, hipStream_t s);
 int launch_build_pairs(const int32_t* topk_ids, const float* topk_w, int T, int k,
                        int E, int S, int32_t* pair_ids, float* pair_w, hipStream_t s);

@@ -375,6 +375,16 @@ __device__ __forceinline__ float from_upper_half(float v) {
     return __uint_as_float(s1);
 }
 
+// Routing weight of a selected expert: its softmax value p, divided by the
+// selected ones' sum (flags & kRenorm), times scaling; rounded to bf16 with
+// kWeightsBf16 (top-k weights cast to the dtype of bf16 router logits,
+// vllm_lut/moe_layer.py:358-376).
+constexpr int kRenorm = 1, kWeightsBf16 = 2;
+__device__ __forceinline__ float routed_weight(float p, float wsum, int flags, float scaling) {
+    const float w = ((flags & kRenorm) ? p / wsum : p) * scaling;
+    return (flags & kWeightsBf16) ? bf16_to_f32(f32_to_bf16(w)) : w;
+}
+
 // Lanes of this wave holding the same id as this lane (ids < 2^nbits;
 // invalid lanes match nobody and get 0): one ballot per id bit.
 __device__ __forceinline__ uint64_t match_lanes(int id, bool ok, int nbits) {

@@ -26,20 +26,28 @@ namespace {
 // One wave per token: lane l holds logits l, l+64, ... (E <= 4096: one bit
 // per held logit in a 64-bit mask); softmax in fp32; top-k by logit (softmax
 // is monotone), ties to the lower expert id.
-__global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits,
+// Logits fp32, or bf16 (kBf16).
+template <bool kBf16>
+__device__ __forceinline__ float logit(const void* p, int64_t i) {
+    return kBf16 ? bf16_to_f32(((const uint16_t*)p)[i]) : ((const float*)p)[i];
+}
+
+template <bool kBf16>
+__global__ __launch_bounds__(256) void route_topk_kernel(const void* __restrict__ logits,
                                                          int T, int E, int k, int renorm,
                                                          float scaling, float* __restrict__ w,
                                                          int32_t* __restrict__ ids) {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= T) return;
-    const float* l = logits + (int64_t)t * E;
+    const int64_t l0 = (int64_t)t * E;
+    auto l = [&](int e) __attribute__((always_inline)) { return logit<kBf16>(logits, l0 + e); };
     float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, l[e]);
+    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, l(e));
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
     float sum = 0.f;
-    for (int e = lane; e < E; e += 64) sum += expf(l[e] - mx);
+    for (int e = lane; e < E; e += 64) sum += expf(l(e) - mx);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, kWave);
     uint64_t taken = 0;
@@ -50,7 +58,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
         int bi = 0x7fffffff;
         int q = 0;
         for (int e = lane; e < E; e += 64, ++q) {
-            const float v = l[e];
+            const float v = l(e);
             if (!((taken >> q) & 1ull) && (v > bv || (v == bv && e < bi))) { bv = v; bi = e; }
         }
 #pragma unroll
@@ -67,8 +75,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
         if (lane == j) { wsel = p; isel = none ? -1 : bi; }
     }
     if (lane < k) {
-        const float v = renorm ? wsel / wsum : wsel;
-        w[(int64_t)t * k + lane] = v * scaling;
+        w[(int64_t)t * k + lane] = routed_weight(wsel, wsum, renorm, scaling);
         ids[(int64_t)t * k + lane] = isel;
     }
 }
@@ -78,13 +85,14 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
 // largest order-preserving key; the lowest lane holding it wins (ties ->
 // lower expert id; -0 == +0; NaN is never selected, and a round with only
 // NaN left yields id -1 and weight 0).
-__global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __restrict__ logits, int T, int E,
-                                                              int k, int renorm, float scaling,
+template <bool kBf16>
+__global__ __launch_bounds__(256) void route_topk_wave_kernel(const void* __restrict__ logits, int T, int E, int k,
+                                                              int renorm, float scaling,
                                                               float* __restrict__ w, int32_t* __restrict__ ids) {
     const int lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= T) return;
-    const float v = lane < E ? logits[(int64_t)t * E + lane] : -INFINITY;
+    const float v = lane < E ? logit<kBf16>(logits, (int64_t)t * E + lane) : -INFINITY;
     const float mx = wave_reduce_max(v);
     const float sum = wave_reduce(lane < E ? expf(v - mx) : 0.f);
     int key = lane < E ? float_key(v) : INT_MIN;
@@ -104,8 +112,7 @@ __global__ __launch_bounds__(256) void route_topk_wave_kernel(const float* __res
         if (lane == sel) key = INT_MIN;
     }
     if (lane < k) {
-        const float x = renorm ? wsel / wsum : wsel;
-        w[(int64_t)t * k + lane] = x * scaling;
+        w[(int64_t)t * k + lane] = routed_weight(wsel, wsum, renorm, scaling);
         ids[(int64_t)t * k + lane] = isel;
     }
 }
@@ -416,15 +423,22 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 
 namespace lutmoe_host {
 
-int launch_route_topk(const float* logits, int T, int E, int k, int renorm, float scaling,
-                      float* w, int32_t* ids, hipStream_t s) {
+template <bool kBf16>
+static int route_topk_dispatch(const void* logits, int T, int E, int k, int renorm, float scaling, float* w,
+                               int32_t* ids, hipStream_t s) {
     if (E <= 64 && k <= 64)
-        hipLaunchKernelGGL(route_topk_wave_kernel, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, E, k, renorm,
+        hipLaunchKernelGGL(route_topk_wave_kernel<kBf16>, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, E, k, renorm,
                            scaling, w, ids);
     else
-        hipLaunchKernelGGL(route_topk_kernel, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, E,
+        hipLaunchKernelGGL(route_topk_kernel<kBf16>, dim3((T + 3) / 4), dim3(256), 0, s, logits, T, E,
                            k, renorm, scaling, w, ids);
     return check_launch();
+}
+
+int launch_route_topk(const void* logits, bool logits_bf16, int T, int E, int k, int renorm, float scaling,
+                      float* w, int32_t* ids, hipStream_t s) {
+    return logits_bf16 ? route_topk_dispatch<true>(logits, T, E, k, renorm, scaling, w, ids, s)
+                       : route_topk_dispatch<false>(logits, T, E, k, renorm, scaling, w, ids, s);
 }
 
 int launch_build_pairs(const int32_t* topk_ids, const float* topk_w, int T, int k, int E,

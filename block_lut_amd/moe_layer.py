@@ -66,6 +66,7 @@ class LUTMoELayer(nn.Module):
     slots of the same stacks, and/or MoEWeights.dense_shared in bf16)."""
 
     ROUTER_KERNEL_MAX_T = 64   # decode batches: the gate kernel; larger: torch's GEMM
+    LOGITS_MAX_E = 320         # routed experts that the layer call routes from logits
 
     def __init__(self, moe: MoEWeights, gate_weight: torch.Tensor, top_k: int,
                  renormalize: bool = False, routed_scaling_factor: float = 1.0,
@@ -84,11 +85,16 @@ class LUTMoELayer(nn.Module):
 
     def router_logits(self, xb: torch.Tensor) -> torch.Tensor:
         """fp32 [T, E] logits of the gate; bf16-rounded values in bf16 router mode."""
+        return self._logits(xb).float()
+
+    def _logits(self, xb: torch.Tensor) -> torch.Tensor:
+        """router_logits in the dtype they are computed in: bf16 from torch's GEMM in bf16
+        router mode, else fp32."""
         bf16 = self.router_dtype == torch.bfloat16
         if xb.shape[0] <= self.ROUTER_KERNEL_MAX_T:
             return ops.router_logits(xb, self.gate, round_bf16=bf16)
         if bf16:
-            return F.linear(xb, self.gate).float()
+            return F.linear(xb, self.gate)
         if self._gate_f32 is None or self._gate_f32.device != self.gate.device:
             self._gate_f32 = self.gate.detach().float()
         return F.linear(xb.float(), self._gate_f32)
@@ -97,17 +103,19 @@ class LUTMoELayer(nn.Module):
         shape = hidden_states.shape
         x = hidden_states.reshape(-1, shape[-1])
         xb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16)).contiguous()
-        logits = self.router_logits(xb)
+        logits = self._logits(xb)
         need = ops.moe_workspace_bytes(self.moe, xb.shape[0], self.top_k)
         if self._ws is None or self._ws.numel() < need or self._ws.device != xb.device:
             self._ws = ops.new_workspace(self.moe, xb.shape[0], self.top_k, xb.device)
-        if self.router_dtype == torch.float32:
-            # top-k from the logits inside the layer kernels
+        bf16 = self.router_dtype == torch.bfloat16
+        if not bf16 or self.moe.num_routed <= self.LOGITS_MAX_E:
+            # top-k from the logits inside the layer kernels; bf16 router: the reference's
+            # _routing, weights cast to the logits dtype
             out = ops.moe_forward_logits(self.moe, xb, logits, self.top_k,
                                          renormalize=self.renormalize,
-                                         scaling=self.routed_scaling_factor, workspace=self._ws)
+                                         scaling=self.routed_scaling_factor, workspace=self._ws,
+                                         bf16_weights=bf16)
         else:
-            # the reference's _routing: softmax top-k, weights cast to the logits dtype
             w, ids = ops.route_topk(logits, self.top_k, renormalize=self.renormalize,
                                     scaling=self.routed_scaling_factor)
             out = ops.moe_forward(self.moe, xb, w.to(torch.bfloat16).float(), ids, workspace=self._ws)

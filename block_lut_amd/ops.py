@@ -262,7 +262,7 @@ def moe_forward(moe: MoEWeights, x: torch.Tensor, topk_weights: torch.Tensor,
         out_dtype = out.dtype
     need = moe_workspace_bytes(moe, T, k)
     if workspace is None or workspace.numel() < need:
-        workspace = new_workspace(moe, T, k, x.device)
+        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)   # (needs no zeroing)
     d = moe.desc()
     N.check("lutmoe_moe_forward",
             N.lib().lutmoe_moe_forward_stages(ctypes.byref(d), x.data_ptr(), w.data_ptr(),
@@ -276,14 +276,18 @@ def moe_forward_logits(moe: MoEWeights, x: torch.Tensor, logits: torch.Tensor, t
                        renormalize: bool = False, scaling: float = 1.0,
                        out: Optional[torch.Tensor] = None, out_dtype: torch.dtype = torch.bfloat16,
                        path: int = PATH_AUTO, workspace: Optional[torch.Tensor] = None,
-                       stages: int = N.STAGE_ALL) -> torch.Tensor:
-    """MoE block forward from router logits: softmax(fp32) -> top-k -> layer."""
+                       stages: int = N.STAGE_ALL, bf16_weights: bool = False) -> torch.Tensor:
+    """MoE block forward from router logits: softmax(fp32) -> top-k -> layer.  ``bf16_weights``
+    rounds the routed weights to bf16 (a bf16 router's top-k weights)."""
     _dev(x, torch.bfloat16, "x")
     T, H = x.shape
     if H != moe.hidden:
         raise ValueError(f"x has {H} features, layer expects {moe.hidden}")
-    lg = logits if logits.dtype == torch.float32 else logits.float()
-    lg = _dev(lg.contiguous(), torch.float32, "logits")
+    # bf16 logits go to the top-k kernel as they are where it runs by itself (more than 64
+    # tokens on the MFMA path); the decode kernels read fp32
+    lg16 = logits.dtype == torch.bfloat16 and T > 64 and path != PATH_GEMV
+    lg = logits if lg16 or logits.dtype == torch.float32 else logits.float()
+    lg = _dev(lg.contiguous(), lg.dtype, "logits")
     if tuple(lg.shape) != (T, moe.num_routed):
         raise ValueError(f"logits must be [T, {moe.num_routed}]")
     if out is None:
@@ -293,13 +297,15 @@ def moe_forward_logits(moe: MoEWeights, x: torch.Tensor, logits: torch.Tensor, t
         out_dtype = out.dtype
     need = moe_workspace_bytes(moe, T, top_k)
     if workspace is None or workspace.numel() < need:
-        workspace = new_workspace(moe, T, top_k, x.device)
+        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)   # (needs no zeroing)
     d = moe.desc()
+    flags = ((N.ROUTE_RENORM if renormalize else 0) | (N.ROUTE_BF16_WEIGHTS if bf16_weights else 0) |
+             (N.ROUTE_BF16_LOGITS if lg16 else 0))
     N.check("lutmoe_moe_forward_logits",
-            N.lib().lutmoe_moe_forward_logits(ctypes.byref(d), x.data_ptr(), lg.data_ptr(), T, top_k,
-                                              int(bool(renormalize)), float(scaling), out.data_ptr(),
-                                              _out_code(out_dtype), workspace.data_ptr(),
-                                              workspace.numel(), path, stages, _stream()))
+            N.lib().lutmoe_moe_forward_logits_ex(ctypes.byref(d), x.data_ptr(), lg.data_ptr(), T, top_k,
+                                                 flags, float(scaling), out.data_ptr(),
+                                                 _out_code(out_dtype), workspace.data_ptr(),
+                                                 workspace.numel(), path, stages, _stream()))
     return out
 
 

@@ -318,6 +318,20 @@ int lutmoe_moe_forward_logits(const lutmoe_moe_desc* d, const void* x_dev, const
                               int out_dtype, void* workspace_dev, size_t workspace_bytes,
                               int force_path, int stages, void* stream);
 
+/* lutmoe_moe_forward_logits with flags, for a bf16 router (the vLLM layer's,
+ * vllm_lut/moe_layer.py:301-304, 358-376), whose top-k weights are cast to the
+ * logits' dtype: LUTMOE_ROUTE_RENORM as `renormalize`,
+ * LUTMOE_ROUTE_BF16_WEIGHTS rounds each routed weight to bf16 (after the
+ * renormalisation and scaling), LUTMOE_ROUTE_BF16_LOGITS reads logits_dev as
+ * bf16 [T][E] (T > 64 on the MFMA path only, else LUTMOE_EUNSUPPORTED). */
+#define LUTMOE_ROUTE_RENORM        1
+#define LUTMOE_ROUTE_BF16_WEIGHTS  2
+#define LUTMOE_ROUTE_BF16_LOGITS   4
+int lutmoe_moe_forward_logits_ex(const lutmoe_moe_desc* d, const void* x_dev, const void* logits_dev,
+                                 int T, int k, int flags, float scaling, void* out_dev, int out_dtype,
+                                 void* workspace_dev, size_t workspace_bytes, int force_path, int stages,
+                                 void* stream);
+
 /* ---- measurement ---------------------------------------------------------- */
 
 /* The HBM floor of the one-token BL4 layer (no counterpart in the reference;

@@ -1652,3 +1652,29 @@ def test_dense_shared_expert_shapes(gpu, T, H, Is):
     bound = ((act.abs() * 2.0 ** -8).pow(2) @ d2.double().pow(2).T).sqrt() * w * 4 + 1e-5 * ref.abs().max()
     assert ((out - ref).abs() <= bound).all()
     assert ((out - ref).norm() / ref.norm()) < 1e-3
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 33, 65])
+@pytest.mark.parametrize("E,renorm", [(12, False), (60, True), (130, False)])
+def test_forward_logits_bf16_router(gpu, T, E, renorm):
+    """A bf16 router's routing inside the layer call (weights rounded to bf16; past 64 tokens
+    the logits read as bf16) against the top-k kernel, the cast and the layer from ids, with
+    ties between the bf16 logits.  E <= 64: the same bits; above, the softmax sums in another
+    order, so a weight may round to its neighbour (2^-8 of it)."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    S, k, H, I = 1, 4, 256, 128
+    w13, w2 = _moe_case("bl4", E, S, H, I, seed=31 + E)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, S)
+    rng = np.random.default_rng(T + E)
+    x = to_dev_bf16(_x(rng, T, H), gpu)
+    lg = torch.from_numpy(rng.standard_normal((T, E)).astype(np.float32)).to(gpu).to(torch.bfloat16)
+    out = ops.moe_forward_logits(moe, x, lg, k, renormalize=renorm, scaling=1.5, out_dtype=torch.float32,
+                                 bf16_weights=True)
+    w, ids = ops.route_topk(lg, k, renormalize=renorm, scaling=1.5)
+    ref = ops.moe_forward(moe, x, w.to(torch.bfloat16).float(), ids, out_dtype=torch.float32)
+    if E <= 64:
+        assert torch.equal(out, ref)
+    else:
+        assert rel_maxabs(out.cpu().numpy(), ref.cpu().numpy()) <= 2.0 ** -8
