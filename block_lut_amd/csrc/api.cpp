@@ -405,6 +405,37 @@ size_t lutmoe_moe_workspace_size(const lutmoe_moe_desc* d, int T, int k) {
 
 namespace lutmoe_host {
 
+// Work items of the stream kernels: at most one short one per expert that has
+// positions beside the full ones.
+static int stream_max_chunks(int64_t P, int E_tot, int positions) {
+    return (int)(P / positions + (P < E_tot ? P : E_tot));
+}
+
+// Positions per work item of the stream.hip projections, 0: not taken.  By the
+// average positions of an active expert (at most; Qwen / DeepSeek / Mixtral
+// shapes and small ones, MI355X, us a layer, stream against the other path):
+//  * past about 27 an item's weights are read and looked up again for its
+//    second 32 positions, and the 256-row tiles of the ring kernels win (26.7:
+//    174 / 202, 32: 520 / 427);
+//  * up to 10, items of 16 positions (of 32: 8.5 144 / 149, 17 189 / 158);
+//  * decode, BL4: the one- and two-token passes read rows in order and win
+//    while most experts hold one position (1.07: 95 / 91, 1.27: 97 / 99, 2.1:
+//    120 / 145); NestedLUT from 18 pairs (16: 26 / 24, 24: 54 / 54, 48: 65 / 72),
+//    REF from 6 (3: 37 / 32, 6: 37 / 40, 76: 108 / 143).
+static int stream_positions(const lutmoe_moe_desc* d, int T, int ke, bool gemv) {
+    const int E_tot = d->num_routed + d->num_shared;
+    const int64_t P = (int64_t)T * ke, experts = P < E_tot ? P : E_tot;
+    if (T <= 2 || E_tot > 512 || P > 27 * experts || !stream_supported(d)) return 0;
+    const int n = P > 10 * experts ? 32 : 16;
+    if (stream_max_chunks(P, E_tot, n) > lutmoe::kMaxChunks) return 0;
+    if (!gemv) return n;
+    switch (d->w13.format) {
+        case LUTMOE_FMT_BL4: return 5 * P >= 7 * experts ? n : 0;
+        case LUTMOE_FMT_NESTED: return P >= 18 ? n : 0;
+        default: return P >= 6 ? n : 0;
+    }
+}
+
 // Shared body of the MoE entry points.  Exactly one of (topk_w, topk_ids) and
 // logits is given.
 int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_w,
@@ -441,6 +472,9 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
         gemv = false;
     }
 
+    // few positions per expert: the projections of stream.hip
+    const int stream_n = gemv || force_path == 0 ? stream_positions(d, T, ke, gemv) : 0;
+
     char* ws = (char*)workspace;
     uint16_t* act = (uint16_t*)(ws + L.act);
     hipStream_t s = stream_of(stream);
@@ -460,7 +494,8 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     if (gemv) {
         // routing + permutation happen inside both decode kernels
         return launch_decode_v2(d, (const uint16_t*)x, topk_w, topk_ids, (const float*)logits, T, k, renorm,
-                                scaling, act, ws + L.route, (float*)(ws + L.y), out, out_dtype, stages, s, addend);
+                                scaling, act, ws + L.route, (float*)(ws + L.y), out, out_dtype, stages, s, addend,
+                                stream_n, (int)prefill_y_splits(P, d->hidden));
     }
     int32_t* pair_ids = (int32_t*)(ws + L.pair_ids);
     float* pair_w = (float*)(ws + L.pair_w);
@@ -484,12 +519,24 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
             topk_ids = ti;
         }
         if ((rc = launch_route_pairs(topk_ids, topk_w, T, k, E, S, (int32_t*)r.offsets, (int32_t*)r.perm,
-                                     (int32_t*)r.inv, (int32_t*)r.active, pair_ids, pair_w, s, r.sched)))
+                                     (int32_t*)r.inv, (int32_t*)r.active, pair_ids, pair_w, s, r.sched,
+                                     stream_n ? (lutmoe::RouteChunks*)(ws + L.route) : nullptr, stream_n)))
             return rc;
         if (d->shared_gate && S > 0 &&
             (rc = launch_shared_gate((const uint16_t*)x, (const uint16_t*)d->shared_gate, T, d->hidden, k, S,
                                      pair_w, s)))
             return rc;
+    }
+    if (stream_n) {
+        const StreamRoute sr{(const lutmoe::RouteChunks*)(ws + L.route), r.perm, nullptr, pair_w, ke,
+                             stream_max_chunks(P, E_tot, stream_n), stream_n};
+        if ((stages & LUTMOE_STAGE_GATE_UP) && (rc = launch_stream_gate_up(d, (const uint16_t*)x, sr, act, s)))
+            return rc;
+        if (!(stages & LUTMOE_STAGE_DOWN)) return LUTMOE_OK;
+        int ns = 1;
+        const int64_t stride = P * d->hidden;
+        if ((rc = launch_stream_down(d, act, sr, y, stride, (int)prefill_y_splits(P, d->hidden), &ns, s))) return rc;
+        return launch_combine(y, r.inv, T, ke, d->hidden, out, out_dtype, s, ns, stride, addend, naddend);
     }
     if ((stages & LUTMOE_STAGE_GATE_UP) &&
         (rc = launch_prefill_gate_up(d, (const uint16_t*)x, r, act, (int)P, s)))

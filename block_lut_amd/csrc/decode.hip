@@ -65,12 +65,7 @@ struct RouteOut {
 // per slot.  NestedLUT at two tokens a pass: C = TB (one pass a chunk; its
 // register lookups make a chunk's weights cheaper to read again than to look
 // up twice).  Stored in the workspace right after the RouteOut copy.
-struct RouteChunks {
-    int nchunk;
-    int ce[kMaxP];                      // expert of chunk c
-    int cp0[kMaxP];                     // its first position
-    int cn[kMaxP];                      // its positions
-};
+static_assert(kMaxChunks == kMaxP, "at most one chunk per pair");
 
 // The routing weight of each position (pw[perm[p]]), stored after the
 // RouteChunks of the global copy: a down-projection wave that knows its first
@@ -100,6 +95,7 @@ struct DecodeArgs {
     const float* logits;       // [T][E] fp32 (logits mode: topk_ids == nullptr)
     int T, k, renorm;          // renorm: kRenorm | kWeightsBf16
     int tb;                    // tokens per pass of the expert loops (1, 2 or 4)
+    int chunk;                 // positions per work item (0: by tb)
     float scaling;
     uint16_t* act;             // [P][I] bf16
     void* out;
@@ -568,7 +564,8 @@ __device__ __forceinline__ void put_chunks(const DecodeArgs& A, const RouteOut& 
     const int TB = A.tb;   // tokens per pass
     const int pv = nact > 0 ? R.aoff[nact - 1] + R.an[nact - 1] : 0;
     const int navg = nact > 0 ? (pv + nact - 1) / nact : 1;
-    const int C = A.d.w13.format == LUTMOE_FMT_NESTED && TB == 2 ? TB : TB * max(1, (navg + TB / 2) / TB);
+    const int C = A.chunk ? A.chunk
+                  : A.d.w13.format == LUTMOE_FMT_NESTED && TB == 2 ? TB : TB * max(1, (navg + TB / 2) / TB);
     const int n = tid < nact ? R.an[tid] : 0;
     const int nc = (n + C - 1) / C;
     const int incl = wave_scan_incl(nc);
@@ -2178,7 +2175,7 @@ int launch_decode_stream_probe(const lutmoe_moe_desc* d, const int32_t* ids, int
 int launch_decode_v2(const lutmoe_moe_desc* d, const uint16_t* x, const float* topk_w,
                      const int32_t* topk_ids, const float* logits, int T, int k, int renorm,
                      float scaling, uint16_t* act, void* route_ws, float* y_ws, void* out,
-                     int out_dtype, int stages, hipStream_t s, const float* addend) {
+                     int out_dtype, int stages, hipStream_t s, const float* addend, int stream, int y_splits) {
     DecodeArgs A{};
     A.addend = addend;
     A.d = *d;
@@ -2204,10 +2201,23 @@ int launch_decode_v2(const lutmoe_moe_desc* d, const uint16_t* x, const float* t
     const int fmt_idx = nested ? 1 : d->w13.format == LUTMOE_FMT_REF ? 2 : 0;
     const int tb = tb_for(T, fmt_idx, P, E_tot);
     A.tb = tb;   // before the routing launch: its chunking reads it
+    A.chunk = stream;
     int rc;
     if (pre && (stages & LUTMOE_STAGE_ROUTE)) {
         hipLaunchKernelGGL(decode_route_kernel, dim3(1), dim3(1024), 0, s, A);
         if ((rc = check_launch())) return rc;
+    }
+    if (stream) {
+        RouteOut* g = A.route;
+        RouteChunks* ch = reinterpret_cast<RouteChunks*>(g + 1);
+        const StreamRoute r{ch, g->perm, reinterpret_cast<RoutePosW*>(ch + 1)->w, nullptr, k + d->num_shared,
+                            std::min(P, max_active + P / stream), stream};
+        if ((stages & LUTMOE_STAGE_GATE_UP) && (rc = launch_stream_gate_up(d, x, r, act, s))) return rc;
+        if (!(stages & LUTMOE_STAGE_DOWN)) return LUTMOE_OK;
+        int ns = 1;
+        const int64_t stride = (int64_t)P * d->hidden;
+        if ((rc = launch_stream_down(d, act, r, y_ws, stride, y_splits, &ns, s))) return rc;
+        return launch_combine(y_ws, g->inv, T, k + d->num_shared, d->hidden, out, out_dtype, s, ns, stride, addend);
     }
 #define LUTMOE_DECODE_CASE(N, TB, PRE, FMT, KERNEL, GRID, BLOCK, LDS) \
     case N: hipLaunchKernelGGL((KERNEL<TB, PRE, FMT>), GRID, BLOCK, LDS, s, A); break;

@@ -6,6 +6,20 @@
 
 #include "../../include/lutmoe.h"
 
+namespace lutmoe {
+
+// Work items of the kernels that take an expert's positions in pieces: item c
+// is positions [cp0, cp0 + cn) of expert ce (device memory, in the workspace).
+constexpr int kMaxChunks = 512;
+struct RouteChunks {
+    int nchunk;
+    int ce[kMaxChunks];
+    int cp0[kMaxChunks];
+    int cn[kMaxChunks];
+};
+
+}  // namespace lutmoe
+
 namespace lutmoe_host {
 
 // noalloc.hip: the device scratch of lutmoe_moe_forward_noalloc, per GPU
@@ -70,11 +84,31 @@ void set_last_error_text(const char* text);
 // decode.hip (BL4 decode layer, routing recomputed inside each CTA)
 bool decode_v2_supported(const lutmoe_moe_desc* d, int T, int k);
 size_t decode_route_bytes();
-// addend: NULL or fp32 [T][H] added to each output before its rounding
+// addend: NULL or fp32 [T][H] added to each output before its rounding;
+// stream: 0, or the positions per work item of the stream.hip projections,
+// which then take the place of the GEMV kernels (y_ws holds y_splits results)
 int launch_decode_v2(const lutmoe_moe_desc* d, const uint16_t* x, const float* topk_w,
                      const int32_t* topk_ids, const float* logits, int T, int k, int renorm,
                      float scaling, uint16_t* act, void* route_ws, float* y_ws, void* out,
-                     int out_dtype, int stages, hipStream_t s, const float* addend = nullptr);
+                     int out_dtype, int stages, hipStream_t s, const float* addend = nullptr, int stream = 0, int y_splits = 1);
+
+// stream.hip: the expert projections for few positions per expert.  The
+// work items hold at most `positions` (16 or 32) positions each.
+struct StreamRoute {
+    const lutmoe::RouteChunks* chunks;
+    const int32_t* perm;      // [P] pair index at each position
+    const float* pos_w;       // [P] routing weight of each position, or NULL:
+    const float* pair_w;      // [P] routing weight of each pair
+    int ke;                   // pairs per token
+    int max_chunks;           // grid bound on chunks->nchunk
+    int positions;
+};
+bool stream_supported(const lutmoe_moe_desc* d);
+int launch_stream_gate_up(const lutmoe_moe_desc* d, const uint16_t* x, const StreamRoute& r, uint16_t* act,
+                          hipStream_t s);
+// y: *nsplit <= max_split partial results (K splits), `stride` floats apart
+int launch_stream_down(const lutmoe_moe_desc* d, const uint16_t* act, const StreamRoute& r, float* y, int64_t stride,
+                       int max_split, int* nsplit, hipStream_t s);
 
 // dense.hip: a dense bf16 shared expert (d->dense_inter > 0).  gate_up:
 // tokw[t] = the shared weight of token t, act [T][Is] bf16; down: y [T][H]
@@ -102,10 +136,12 @@ int launch_build_pairs(const int32_t* topk_ids, const float* topk_w, int T, int 
 int launch_permute(const int32_t* pair_ids, int T, int k_eff, int E_tot, int32_t* offsets,
                    int32_t* perm, int32_t* inv, int32_t* active, hipStream_t s);
 // pairs built from top-k ids (+ S shared slots per token), permuted, and
-// their ids / weights written to pair_ids / pair_w
+// their ids / weights written to pair_ids / pair_w; with chunks (E + S <= 512),
+// every expert's positions cut into work items of at most `chunk`
 int launch_route_pairs(const int32_t* topk_ids, const float* topk_w, int T, int k, int E, int S,
                        int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* active, int32_t* pair_ids,
-                       float* pair_w, hipStream_t s, int32_t* sched = nullptr);
+                       float* pair_w, hipStream_t s, int32_t* sched = nullptr,
+                       lutmoe::RouteChunks* chunks = nullptr, int chunk = 0);
 // shared slots k..k+S-1 of every token t: pair_w = sigmoid(x_t . gate)
 int launch_shared_gate(const uint16_t* x, const uint16_t* gate, int T, int H, int k, int S, float* pair_w,
                        hipStream_t s);

@@ -185,8 +185,12 @@ __device__ __forceinline__ u32x4_t regtab_lookup8_eo(const uint32_t* lo, const u
     if constexpr (B == 4) {
         se7 = se & 0x07070707u;
         so7 = so & 0x07070707u;
-        sel_e = ((se >> 1) & 0x04040404u) | 0x03020100u;
-        sel_o = ((so >> 1) & 0x04040404u) | 0x03020100u;
+        // the constants in registers: a shift and one v_and_or_b32 each
+        uint32_t bit, idx;
+        asm("s_mov_b32 %0, 0x04040404" : "=s"(bit));
+        asm("v_mov_b32 %0, 0x03020100" : "=v"(idx));
+        sel_e = ((w >> 1) & bit) | idx;
+        sel_o = ((w >> 5) & bit) | idx;
     }
     const uint32_t le = plane_lookup4<B>(lo, se, se7, sel_e), he = plane_lookup4<B>(hi, se, se7, sel_e);
     const uint32_t lo_ = plane_lookup4<B>(lo, so, so7, sel_o), ho = plane_lookup4<B>(hi, so, so7, sel_o);

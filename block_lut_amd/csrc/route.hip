@@ -271,7 +271,8 @@ __global__ __launch_bounds__(1024) void permute_chunk_kernel(PairSrc ps, int P, 
                                                              int32_t* __restrict__ active,
                                                              int32_t* __restrict__ pair_ids,
                                                              float* __restrict__ pair_w,
-                                                             int32_t* __restrict__ sched) {
+                                                             int32_t* __restrict__ sched,
+                                                             RouteChunks* __restrict__ chunks, int chunk) {
     extern __shared__ int32_t sm[];   // h_all[E_tot] | h_bef[E_tot] | off[E_tot+1] | sub[kPermSub][E_tot]
     int32_t* h_all = sm;
     int32_t* h_bef = sm + E_tot;
@@ -329,10 +330,28 @@ __global__ __launch_bounds__(1024) void permute_chunk_kernel(PairSrc ps, int P, 
     // (c) offsets (wave 0: lane l owns experts [l*per, l*per+per)), active list
     if (wv == 0) {
         const int per = (E_tot + 63) / 64;
-        int c = 0, a = 0;
+        int c = 0, a = 0, nw = 0;
         for (int q = 0; q < per; ++q) {
             const int e = lane * per + q;
-            if (e < E_tot) { c += h_all[e]; a += h_all[e] > 0; }
+            if (e < E_tot) {
+                c += h_all[e];
+                a += h_all[e] > 0;
+                if (chunks) nw += (h_all[e] + chunk - 1) / chunk;
+            }
+        }
+        if (chunks && blockIdx.x == 0) {   // work items, experts ascending
+            int p = wave_scan_incl(c) - c, o = wave_scan_incl(nw) - nw;
+            if (lane == 63) chunks->nchunk = o + nw;
+            for (int q = 0; q < per; ++q) {
+                const int e = lane * per + q;
+                const int h = e < E_tot ? h_all[e] : 0;
+                for (int m = 0; m < h; m += chunk, ++o) {
+                    chunks->ce[o] = e;
+                    chunks->cp0[o] = p + m;
+                    chunks->cn[o] = min(chunk, h - m);
+                }
+                p += h;
+            }
         }
         int oc = wave_scan_incl(c) - c, oa = wave_scan_incl(a) - a;
         for (int q = 0; q < per; ++q) {
@@ -471,7 +490,7 @@ int launch_permute(const int32_t* pair_ids, int T, int k_eff, int E_tot, int32_t
 
 int launch_route_pairs(const int32_t* topk_ids, const float* topk_w, int T, int k, int E, int S,
                        int32_t* offsets, int32_t* perm, int32_t* inv, int32_t* active, int32_t* pair_ids,
-                       float* pair_w, hipStream_t s, int32_t* sched) {
+                       float* pair_w, hipStream_t s, int32_t* sched, RouteChunks* chunks, int chunk) {
     const int ke = k + S, E_tot = E + S;
     const int P = T * ke;
     if (E_tot <= 512) {
@@ -481,7 +500,7 @@ int launch_route_pairs(const int32_t* topk_ids, const float* topk_w, int T, int 
         const size_t lds = ((size_t)(3 + kPermSub) * E_tot + 1) * sizeof(int32_t);
         const PairSrc ps{topk_ids, topk_w, T, k, ke, E};
         hipLaunchKernelGGL(permute_chunk_kernel, dim3(nchunk), dim3(64 * kPermSub), lds, s, ps, P, E_tot, nbits,
-                           offsets, perm, inv, active, pair_ids, pair_w, sched);
+                           offsets, perm, inv, active, pair_ids, pair_w, sched, chunks, chunk);
         return check_launch();
     }
     int rc;

@@ -1678,3 +1678,40 @@ def test_forward_logits_bf16_router(gpu, T, E, renorm):
         assert torch.equal(out, ref)
     else:
         assert rel_maxabs(out.cpu().numpy(), ref.cpu().numpy()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("fmt", ["bl4", "ref", "nested"])
+@pytest.mark.parametrize("T,E,k,H,I,skew", [(3, 4, 3, 64, 64, 0), (6, 5, 2, 192, 128, 0), (17, 6, 3, 128, 192, 1),
+                                            (33, 7, 2, 2112, 64, 0), (40, 4, 2, 256, 1088, 1), (50, 3, 1, 4224, 64, 2),
+                                            (70, 12, 4, 320, 448, 1)])
+def test_moe_layer_few_positions_per_expert(gpu, fmt, T, E, k, H, I, skew):
+    """The weight-streaming projections (stream.hip) at their edges, the layer against the
+    oracle: items of 16 and 32 positions, full, left over and cut from one heavy expert
+    (skew), dropped pairs, K of one and more 128-column steps with a last one of 64, more
+    columns than LDS holds of the activations, a K long enough for its two splits, half a
+    CTA's rows; decode and prefill routing."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    rng = np.random.default_rng(T * H + I)
+    if fmt == "nested":
+        bits = [(2, 3, 4)[e % 3] for e in range(E + 1)]
+        w13 = NestedExpertset(bits, 2 * I, H, seed=700 + T, n_iter=4)
+        w2 = NestedExpertset(bits, H, I, seed=701 + T, n_iter=4)
+    else:
+        w13, w2 = _moe_case(fmt, E, 1, H, I, seed=700 + T)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 1)
+    xb = _x(rng, T, H)
+    lg = rng.standard_normal((T, E)).astype(np.float32)
+    if skew:
+        lg[:, 1] += 6.0                        # one expert on nearly every token
+    rw, rids = O.route(lg, k)
+    if skew == 2:
+        rids = rids.copy()
+        rids[::5] = -1                         # dropped pairs
+    out = ops.moe_forward(moe, to_dev_bf16(xb, gpu), torch.from_numpy(rw).to(gpu), torch.from_numpy(rids).to(gpu),
+                          out_dtype=torch.float32).cpu().numpy()
+    keep = rids >= 0
+    ref = O.moe_layer(xb, np.where(keep, rids, 0), np.where(keep, rw, 0), w13.deq_f32, w2.deq_f32,
+                      shared=[(w13.deq_f32(E), w2.deq_f32(E))])
+    assert rel_maxabs(out, ref) <= TOL
