@@ -1,5 +1,5 @@
 // Grouped LUT-GEMM for few tokens per expert (3 tokens and more, up to about
-// 24 positions an expert): weights streamed straight to registers, looked up
+// 24 positions an expert): weights streamed to registers, looked up
 // there, and multiplied on MFMA (16 x 16 x 32, gfx950).
 //
 // It stands between the decode GEMV kernels, which look every weight up again
@@ -9,10 +9,14 @@
 // weight rows (gate/up: 8 gate and 8 up rows, so the SwiGLU pair meets in one
 // wave) and one work item: up to 16 NM positions of one expert.  Two CTAs a CU,
 // 4 waves a SIMD.
-//   K step: 128 columns.  Lane (n = l % 16, g = l / 16) holds columns 32g ..
+//   K step: 128 columns.  Lane (n = l % 16, g = l / 16) looks up columns 32g ..
 //     32g + 31 of row n: BL4 16 code bytes, NestedLUT one 32-weight group, REF 32
-//     code bytes; its block's table (or absmax) beside them.  The next two
-//     steps are in flight while two are looked up, none of it through LDS.
+//     code bytes; its block's table (or absmax) beside them.  REF loads them
+//     itself.  BL4 / NestedLUT rows are loaded in 16-byte pieces on consecutive
+//     lanes, three steps ahead, and reach their lane through 2 KB of LDS that the
+//     wave has to itself: 16 rows on consecutive lanes cost the address unit a
+//     cache line a lane (Mixtral shape BL4 T = 16 / 64 352 / 385 -> 312 / 364 us
+//     on one card, NestedLUT 283 / 365 -> 270 / 346, Qwen shape 1-4 % less).
 //   Lookups: BL4 / NestedLUT by v_perm over the block's table as byte planes.
 //     REF: the fp32 codebook in LDS, one copy per bank (32 KB, entry c of lane l
 //     at 128 c + 4 (l % 32)): a lookup never meets another lane's bank, where 64
@@ -23,9 +27,9 @@
 // Results leave the accumulators as runs of 4 outputs of one position.
 //
 // Before / here, us a layer (the GEMV kernels up to 32 tokens, the ring above):
-// Qwen shape BL4 T = 32 / 64 / 256 145 / 185 / 195 -> 120 / 130 / 157, REF T = 19 / 64
-// 143 / 231 -> 108 / 144, NestedLUT tiers T = 16 / 64 83 / 183 -> 73 / 111; Mixtral
-// shape BL4 T = 16 / 64 576 / 408 -> 300 / 345 (4.7 TB/s at T = 16).
+// Qwen shape BL4 T = 32 / 64 / 256 145 / 185 / 195 -> 119 / 129 / 155, REF T = 19 / 64
+// 143 / 231 -> 108 / 144, NestedLUT tiers T = 16 / 64 83 / 183 -> 68 / 111; Mixtral
+// shape BL4 T = 16 / 64 576 / 408 -> 299 / 341 (4.7 TB/s at T = 16).
 #include "common.h"
 #include "kernels.h"
 #include "lut_core.h"
@@ -48,69 +52,139 @@ struct StreamArgs {
 // A weight array, uniform and in global memory (pointers that come from memory
 // would otherwise be loaded from with flat loads).
 typedef __attribute__((address_space(1))) const uint8_t* gbytes_t;
-typedef __attribute__((address_space(1))) const uint32_t* gwords_t;
-typedef __attribute__((address_space(1))) const u32x4_t* gquads_t;
+typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));   // (3-bit codes and 2-bit tables: 8-byte aligned)
+typedef __attribute__((address_space(1))) const u32x4_a4_t* gquads_t;
 __device__ __forceinline__ gbytes_t weight_array(const void* p) {
     const uint64_t v = (uint64_t)p;
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (gbytes_t)(((uint64_t)hi << 32) | lo);
 }
-// N dwords at p
-template <int N>
-__device__ __forceinline__ void load_words(uint32_t (&d)[N], gbytes_t p) {
-    if constexpr (N % 4 == 0) {
-#pragma unroll
-        for (int i = 0; i < N; i += 4) {
-            const u32x4_t v = *(gquads_t)(p + 4 * i);
-            d[i] = v[0];
-            d[i + 1] = v[1];
-            d[i + 2] = v[2];
-            d[i + 3] = v[3];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) d[i] = ((gwords_t)p)[i];
-    }
+__device__ __forceinline__ u32x4_t load16(gbytes_t p, uint32_t off) {
+    return *(gquads_t)(p + off);
+}
+__device__ __forceinline__ u32x4_t lds_ld128(uint32_t a) {
+    return *(__attribute__((address_space(3))) const u32x4_t*)a;
+}
+__device__ __forceinline__ void lds_st128(uint32_t a, u32x4_t v) {
+    *(__attribute__((address_space(3))) u32x4_t*)a = v;
 }
 
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// One K step's weights of one lane, and their MFMA fragments.  B: code bits of
-// a table format (BL4: 4).
-template <int kFmt, int B>
-struct Step {
-    static constexpr bool kBl4 = kFmt == LUTMOE_FMT_BL4;
-    static constexpr int kTab = (1 << B) / 2;      // table dwords of a block
-    uint32_t c[B], t[kTab];
+// Keeps a wave-uniform condition a branch (not selects on every path).
+__device__ __forceinline__ void rare_branch() { asm volatile(""); }
 
-    // row_c / row_t: byte offsets of the lane's row; g: lane group (tail: g & 1)
-    __device__ __forceinline__ void load(gbytes_t codes, gbytes_t tabs, uint32_t row_c, uint32_t row_t, int step,
-                                         int g) {
-        const uint32_t co = row_c + (uint32_t)(4 * step + g) * (4 * B);
-        const uint32_t to = row_t + (uint32_t)(2 * step + (g >> 1)) * (4 * kTab);
-        load_words(c, codes + co);
-        load_words(t, tabs + to);
+constexpr int kSlotB = 2048;   // LDS bytes of a wave's K step of weights
+
+// A wave's weights of one K step (16 rows x 128 columns) go global -> registers
+// in 16-byte pieces of a row on consecutive lanes (a load of 16 bytes a lane
+// from 16 different rows on consecutive lanes would take a cache line access
+// per lane), then through the wave's LDS slot to the lane that looks them up:
+// lane (n, g), columns 32g .. 32g + 31 of row n.  B: code bits (BL4: 4).
+template <int B>
+struct Weights {
+    static constexpr int kTab = (1 << B) / 2;   // table dwords of a block
+    static constexpr int CP = B, TP = kTab / 2; // 16-byte pieces of a row's codes / tables per step
+    uint32_t off_c, off_t;      // this lane's pieces, from the step's first byte of the arrays
+    uint32_t wr_c, wr_t;        // their LDS addresses
+    uint32_t rd_c, rd_t[2];     // LDS addresses of lane (n, g)
+    int cp, tp;
+    struct Raw {
+        u32x4_t c, t;
+    };
+    struct Step {
+        uint32_t c[B], t[kTab];
+    };
+    static __device__ __forceinline__ int swz(int r) { return B == 4 ? (r >> 1) & 3 : 0; }
+
+    // row(i): the weight row of the wave's row i
+    template <class RowFn>
+    __device__ __forceinline__ void init(int lane, int K, uint32_t slot, RowFn row) {
+        const int cr = min(lane / CP, 15), tr = min(lane / TP, 15);
+        cp = lane < 16 * CP ? lane % CP : CP - 1;   // (lanes past the pieces repeat the last)
+        tp = lane < 16 * TP ? lane % TP : TP - 1;
+        off_c = row(cr) * (uint32_t)(K / 8 * B) + 16u * (uint32_t)cp;
+        off_t = row(tr) * (uint32_t)(K / 64 * 4 * kTab) + 16u * (uint32_t)tp;
+        wr_c = slot + (uint32_t)(cr * 16 * CP + 16 * (cp ^ swz(cr)));
+        wr_t = slot + 1024u + (uint32_t)(tr * 16 * TP + 16 * (tp ^ swz(tr)));
+        const int n = lane & 15, g = lane >> 4;
+        rd_c = slot + (uint32_t)(n * 16 * CP + (B == 4 ? 16 * (g ^ swz(n)) : 4 * B * g));
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            rd_t[h] = slot + 1024u +
+                      (uint32_t)(n * 16 * TP + (B == 4 ? 16 * ((2 * (g >> 1) + h) ^ swz(n)) : 4 * kTab * (g >> 1)));
+    }
+    // tail: the step has 64 columns; pieces past the row's end start at its last
+    // 16 bytes instead
+    __device__ __forceinline__ void load(Raw& r, gbytes_t codes, gbytes_t tabs, int step, bool tail) const {
+        // offsets from the arrays' starts (never below them: a wrapped 32-bit
+        // offset would point 4 GiB past)
+        uint32_t oc = off_c + (uint32_t)step * (16 * CP), ot = off_t + (uint32_t)step * (16 * TP);
+        if (tail) {
+            rare_branch();
+            oc -= 16u * (uint32_t)cp - (uint32_t)min(16 * cp, 8 * B - 16);
+            if constexpr (B > 2) {
+                ot -= 16u * (uint32_t)tp - (uint32_t)min(16 * tp, 4 * kTab - 16);
+            } else {   // 8 bytes of table left: the 16 that end there (never before the array)
+                ot -= min(ot, 8u);
+            }
+        }
+        r.c = load16(codes, oc);
+        r.t = load16(tabs, ot);
     }
     // the loaded words as values that appear here: the compiler then derives
     // nothing from them (and waits for them) before this point
-    __device__ __forceinline__ void arrive() {
-#pragma unroll
-        for (int i = 0; i < B; ++i) asm volatile("" : "+v"(c[i]));
-#pragma unroll
-        for (int i = 0; i < kTab; ++i) asm volatile("" : "+v"(t[i]));
+    static __device__ __forceinline__ void arrive(Raw& r) { asm volatile("" : "+v"(r.c), "+v"(r.t)); }
+    __device__ __forceinline__ void store(const Raw& r, int step, bool tail) const {
+        uint32_t c = wr_c, t = wr_t;
+        u32x4_t tv = r.t;
+        if (tail) {
+            rare_branch();
+            const int lane = (int)threadIdx.x & 63;
+            const int cr = min(lane / CP, 15), tr = min(lane / TP, 15);
+            const int cs = min(16 * cp, 8 * B - 16);   // byte start within the row's step
+            c = wr_c - (uint32_t)(16 * (cp ^ swz(cr))) + (uint32_t)(B == 4 ? 16 * ((cs >> 4) ^ swz(cr)) : cs);
+            if constexpr (B == 4) {
+                t = wr_t - (uint32_t)(16 * (tp ^ swz(tr))) + (uint32_t)(16 * (min(tp, 1) ^ swz(tr)));
+            } else if constexpr (B == 3) {
+                t = wr_t - 16u * (uint32_t)tp;
+            } else {
+                if (off_t + (uint32_t)step * (16 * TP) >= 8u) tv = u32x4_t{tv[2], tv[3], tv[2], tv[3]};
+            }
+        }
+        lds_st128(c, r.c);
+        lds_st128(t, tv);
     }
-    __device__ __forceinline__ void planes(uint32_t* lo, uint32_t* hi) const { table_planes<B>(t, lo, hi); }
-    __device__ __forceinline__ bf16x8_t frag(const uint32_t* lo, const uint32_t* hi, int j) const {
-        uint32_t w;
-        if constexpr (kBl4) w = c[j];
-        else w = nested_code8<B>(c[0], c[1], B >= 3 ? c[B >= 3 ? 2 : 0] : 0u, B >= 4 ? c[B >= 4 ? 3 : 0] : 0u, j);
-        return __builtin_bit_cast(bf16x8_t, regtab_lookup8_eo<B>(lo, hi, w));
+    __device__ __forceinline__ void read(Step& s) const {
+        if constexpr (B == 4) {
+            const u32x4_t v = lds_ld128(rd_c), t0 = lds_ld128(rd_t[0]), t1 = lds_ld128(rd_t[1]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s.c[i] = v[i];
+                s.t[i] = t0[i];
+                s.t[4 + i] = t1[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < B; ++i) s.c[i] = lds_ld32(rd_c + 4 * i);
+#pragma unroll
+            for (int i = 0; i < kTab; ++i) s.t[i] = lds_ld32(rd_t[0] + 4 * i);
+        }
+    }
+    // code dword of the lane's 8 columns j; kBl4: in column order as stored
+    template <bool kBl4>
+    static __device__ __forceinline__ uint32_t code(const Step& s, int j) {
+        if constexpr (kBl4) return s.c[j];
+        else return nested_code8<B>(s.c[0], s.c[1], B >= 3 ? s.c[B >= 3 ? 2 : 0] : 0u, B >= 4 ? s.c[B >= 4 ? 3 : 0] : 0u, j);
     }
 };
 
+// REF: 32 code bytes of its row a lane and step, straight to the lane that looks
+// them up (a row's step is a whole cache line; through the slot was no faster,
+// and slower where the codebook's lookups already fill the LDS).
 struct RefStep {
     u32x4_t c[2];
     uint32_t am;
@@ -152,6 +226,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
     constexpr int KS = KC / 128;                    // their K steps
     static_assert(KS % 4 == 0, "a staging holds whole rounds of the K loop");
     __shared__ __attribute__((aligned(16))) uint8_t s_x[KC * 16 * NM * 2];
+    __shared__ __attribute__((aligned(16))) uint8_t s_w[kRef ? 16 : kWaves * kSlotB];
     __shared__ __attribute__((aligned(16))) float s_cb[kRef ? 256 * 32 : 4];
     const RouteChunks* ch = A.r.chunks;
     const int item = blockIdx.y;
@@ -167,10 +242,11 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
     const int nst_all = (K + 127) / 128, st0 = nst_all * (int)blockIdx.z / (int)gridDim.z;
     const int nst = nst_all * ((int)blockIdx.z + 1) / (int)gridDim.z - st0;
     const bool half_tail = (K & 64) != 0;   // the last step has 64 columns: groups 2, 3 past K
-    // first output of the wave, and this lane's weight row
+    // first output of the wave, and the weight row of its row i
     const int o0 = (int)blockIdx.x * (kGateUp ? 64 : 128) + wv * (kGateUp ? 8 : 16);
-    const uint32_t row = kGateUp ? (uint32_t)min(ln < 8 ? o0 + ln : I + o0 + ln - 8, M - 1)
-                                 : (uint32_t)min(o0 + ln, M - 1);
+    auto row = [&](int i) __attribute__((always_inline)) {
+        return (uint32_t)min(!kGateUp ? o0 + i : i < 8 ? o0 + i : I + o0 + i - 8, M - 1);
+    };
     f32x4_t acc[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -222,21 +298,55 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
             acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc[m], 0, 0, 0);
         }
     };
-    // the K loop: load(buffer, step, group), use(buffer, step, last step of 64).
-    // Steps go in pairs (256 columns: a pair's loads touch whole 128-byte lines
-    // of a row together), the next pair's loads issued before a pair is used.
-    // The loop over pairs that have a next pair has no condition around its
-    // loads, so the compiler's wait counts keep them in flight.
-    // (Steps are counted from st0.)
-    auto k_loop = [&](auto* buf, auto load, auto use) __attribute__((always_inline)) {
+    // Steps are counted from st0; the last one may have 64 columns.
+    auto is_tail = [&](int s) __attribute__((always_inline)) { return half_tail && st0 + s == nst_all - 1; };
+    // BL4 / NestedLUT: load(buffer, step) three steps ahead,
+    // store(buffer, step) to the wave's slot one step ahead (behind the reads of
+    // the step before, which the LDS serves in order), use(step, stored).  Every load
+    // is unconditional (past the end: the last step again), so that the compiler's
+    // wait counts keep them in flight, and the code is one round of 4 steps (the
+    // first pass through it waits for its instructions).
+    auto k_loop_staged = [&](auto* buf, auto load, auto store, auto use) __attribute__((always_inline)) {
+        auto load_step = [&](int b, int s) __attribute__((always_inline)) {
+            const int c = min(s, nst - 1);
+            load(buf[b], st0 + c, is_tail(c));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int q = 0; q < 3; ++q) load_step(q, q);
+        for (int c0 = 0; c0 < nst; c0 += KS) {
+            if (c0) lds_barrier();   // every wave is done with the columns in LDS
+            stage(c0);
+            lds_barrier();
+            if (c0 == 0) store(buf[0], st0, is_tail(0));
+            const int c1 = min(c0 + KS, nst);
+            for (int s0 = c0; s0 < c1; s0 += 4) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int s = s0 + u;
+                    load_step((u + 3) & 3, s + 3);
+                    if (s < c1) {
+                        use(s, is_tail(s), [&]() __attribute__((always_inline)) {
+                            const int c = min(s + 1, nst - 1);
+                            store(buf[(u + 1) & 3], st0 + c, is_tail(c));
+                        });
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+    };
+    // REF: steps in pairs, the next pair's loads issued before a pair is used.  The
+    // loop over pairs that have a next pair has no condition around its loads or
+    // its uses.  (The loop above measured 3-6 % more here.)
+    auto k_loop_pairs = [&](auto* buf, auto load, auto use) __attribute__((always_inline)) {
         auto load_pair = [&](int b, int s) __attribute__((always_inline)) {
             const int a0 = st0 + min(s, nst - 1), a1 = st0 + min(s + 1, nst - 1);
-            load(buf[b], a0, half_tail && a0 == nst_all - 1 ? g & 1 : g);
-            load(buf[b + 1], a1, half_tail && a1 == nst_all - 1 ? g & 1 : g);
+            load(buf[b], a0, is_tail(a0 - st0));
+            load(buf[b + 1], a1, is_tail(a1 - st0));
             __builtin_amdgcn_sched_barrier(0);
         };
         auto use_step = [&](int b, int s, bool tail) __attribute__((always_inline)) {
-            buf[b].arrive();
             use(buf[b], s, tail);
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -261,12 +371,12 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     if (s0 + u >= c1) break;
-                    use_step(u, s0 + u, half_tail && st0 + s0 + u == nst_all - 1);
+                    use_step(u, s0 + u, is_tail(s0 + u));
                 }
             }
         }
     };
-    const bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
+    const uint32_t slot = lds_addr(s_w) + (uint32_t)(wv * kSlotB);
     if constexpr (kRef) {
         {   // the bank-private codebook copies: thread t writes half of entry t / 2
             const float c = bf16_to_f32(ref_codebook(A.w, e)[tid >> 1]);
@@ -277,13 +387,15 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
         const uint8_t* codes = (const uint8_t*)A.w.codes + (int64_t)e * M * K;
         const uint16_t* am = (const uint16_t*)A.w.tables + (int64_t)e * A.w.absmax_per_expert;
         const uint32_t q32 = (uint32_t)A.w.block_size / 32u, nb = (uint32_t)A.w.absmax_per_expert;
-        const uint32_t cbase = lds_addr(s_cb) + 4u * (uint32_t)(lane & 31);
+        const uint32_t cbase = lds_addr(s_cb) + 4u * (uint32_t)(lane & 31), r = row(ln);
+        const bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0u, 0u, 0u, 0u});
         RefStep buf[4];
-        k_loop(buf,
-               [&](RefStep& b, int s, int gg) __attribute__((always_inline)) {
-                   b.load(codes, am, row * (uint32_t)K, row * (uint32_t)(K / 32), q32, nb, s, gg);
+        k_loop_pairs(buf,
+               [&](RefStep& b, int step, bool tail) __attribute__((always_inline)) {
+                   b.load(codes, am, r * (uint32_t)K, r * (uint32_t)(K / 32), q32, nb, step, tail ? g & 1 : g);
                },
                [&](RefStep& b, int s, bool tail) __attribute__((always_inline)) {
+                   b.arrive();
 #pragma unroll
                    for (int j = 0; j < 4; ++j) {
                        bf16x8_t w = b.frag(cbase, j);
@@ -294,20 +406,32 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
     } else {
         auto run = [&](auto BC, gbytes_t codes, gbytes_t tabs) __attribute__((always_inline)) {
             constexpr int B = decltype(BC)::value;
-            using St = Step<kFmt, B>;
-            const uint32_t row_c = row * (uint32_t)(K / 8 * B), row_t = row * (uint32_t)(K / 64 * 4 * St::kTab);
-            St buf[4];
-            k_loop(buf,
-                   [&](St& b, int s, int gg) __attribute__((always_inline)) { b.load(codes, tabs, row_c, row_t, s, gg); },
-                   [&](St& b, int s, bool tail) __attribute__((always_inline)) {
+            using Wt = Weights<B>;
+            Wt W;
+            W.init(lane, K, slot, row);
+            typename Wt::Raw buf[4];
+            k_loop_staged(buf, [&](typename Wt::Raw& b, int step, bool tail) __attribute__((always_inline)) { W.load(b, codes, tabs, step, tail); },
+                   [&](typename Wt::Raw& b, int step, bool tail) __attribute__((always_inline)) {
+                       W.arrive(b);
+                       W.store(b, step, tail);
+                   },
+                   [&](int s, bool tail, auto next) __attribute__((always_inline)) {
+                       typename Wt::Step st;
+                       W.read(st);
+                       next();
                        uint32_t lo[(1 << B) / 4], hi[(1 << B) / 4];
-                       b.planes(lo, hi);
-                       if (tail && g >= 2) {   // lanes past K read another block: zero weights
+                       table_planes<B>(st.t, lo, hi);
+                       if (tail) {   // lanes past K hold other tables: zero weights
+                           rare_branch();
 #pragma unroll
-                           for (int i = 0; i < (1 << B) / 4; ++i) lo[i] = hi[i] = 0u;
+                           for (int i = 0; i < (1 << B) / 4; ++i) {
+                               lo[i] = g >= 2 ? 0u : lo[i];
+                               hi[i] = g >= 2 ? 0u : hi[i];
+                           }
                        }
 #pragma unroll
-                       for (int j = 0; j < 4; ++j) mma(s, j, b.frag(lo, hi, j));
+                       for (int j = 0; j < 4; ++j)
+                           mma(s, j, __builtin_bit_cast(bf16x8_t, regtab_lookup8_eo<B>(lo, hi, Wt::template code<!kNested>(st, j))));
                    });
         };
         if constexpr (kNested) {
