@@ -75,12 +75,16 @@ def measured_traffic(name):
 
 
 def decode_kernel_label(T, P, E_tot):
-    """The gate/up kernel the library launches for this batch (the tokens-per-pass rule of
-    decode.hip's tb_for for BL4: one token its own kernel, two-token passes up to 16
-    tokens, and up to 32 while the experts hold at most 3 positions on average)."""
+    """The gate/up kernel the library launches for this batch (BL4; api.cpp's
+    stream_positions and decode.hip's tb_for): one token its own kernel, the streaming MFMA
+    kernel from 1.4 to 27 positions an active expert, else two-token passes up to 16 tokens
+    (and up to 32 while the experts hold at most 3 positions on average)."""
     if T <= 1:
         return "bl4_decode_gate_up_t1"
-    tb = 2 if T <= 16 or (T <= 32 and P <= 3 * min(P, E_tot)) else 4
+    experts = min(P, E_tot)
+    if T > 2 and E_tot <= 512 and 7 * experts <= 5 * P and P <= 27 * experts:
+        return f"stream_kernel<gate_up, {2 if P > 10 * experts else 1}>"
+    tb = 2 if T <= 16 or (T <= 32 and P <= 3 * experts) else 4
     return f"bl4_decode_gate_up<{tb}>"
 
 
