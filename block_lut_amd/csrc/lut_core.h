@@ -386,7 +386,8 @@ __device__ __forceinline__ float from_upper_half(float v) {
 constexpr int kRenorm = 1, kWeightsBf16 = 2;
 __device__ __forceinline__ float routed_weight(float p, float wsum, int flags, float scaling) {
     const float w = ((flags & kRenorm) ? p / wsum : p) * scaling;
-    return (flags & kWeightsBf16) ? bf16_to_f32(f32_to_bf16(w)) : w;
+    const float b = __uint_as_float(f32x2_to_bf16x2(w, w) << 16);   // (selected: no branch in the route)
+    return (flags & kWeightsBf16) ? b : w;
 }
 
 // Lanes of this wave holding the same id as this lane (ids < 2^nbits;

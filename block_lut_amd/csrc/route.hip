@@ -399,7 +399,7 @@ __global__ __launch_bounds__(1024) void permute_chunk_kernel(PairSrc ps, int P, 
 // are read once: non-temporal loads.  Latency-bound for a decode batch, so one
 // kernel per number of positions KE (k + shared experts), whose loads have no
 // branch between them: a dropped pair (position -1) reads row 0 and adds zero.
-// (Qwen shape T = 8, 5 positions: down and combine 23.95 -> 23.35 us against one
+// (Qwen shape T = 8, 4 positions: down and combine 23.95 -> 23.35 us against one
 // kernel for all KE with a branch around each load.)
 template <int KE>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ y, const int32_t* __restrict__ inv,
