@@ -178,19 +178,23 @@ __device__ __forceinline__ u32x4_t regtab_lookup8(const uint32_t* lo, const uint
 // regtab_lookup8 without its last step: the 8 weights in the order
 // w0, w2, w4, w6, w1, w3, w5, w7 (an MFMA operand whose partner operand holds
 // its 8 k-values in the same order gives the same products)
-template <int B>
+template <int B, bool kConstRegs = false>
 __device__ __forceinline__ u32x4_t regtab_lookup8_eo(const uint32_t* lo, const uint32_t* hi, uint32_t w) {
     const uint32_t se = w & 0x0f0f0f0fu, so = (w >> 4) & 0x0f0f0f0fu;
     uint32_t se7 = se, so7 = so, sel_e = 0, sel_o = 0;
     if constexpr (B == 4) {
         se7 = se & 0x07070707u;
         so7 = so & 0x07070707u;
-        // the constants in registers: a shift and one v_and_or_b32 each
-        uint32_t bit, idx;
-        asm("s_mov_b32 %0, 0x04040404" : "=s"(bit));
-        asm("v_mov_b32 %0, 0x03020100" : "=v"(idx));
-        sel_e = ((w >> 1) & bit) | idx;
-        sel_o = ((w >> 5) & bit) | idx;
+        if constexpr (kConstRegs) {   // a shift and one v_and_or_b32 each
+            uint32_t bit, idx;
+            asm("s_mov_b32 %0, 0x04040404" : "=s"(bit));
+            asm("v_mov_b32 %0, 0x03020100" : "=v"(idx));
+            sel_e = ((w >> 1) & bit) | idx;
+            sel_o = ((w >> 5) & bit) | idx;
+        } else {   // (the ring kernels: DeepSeek T=2048 1 % slower with the two registers taken)
+            sel_e = ((se >> 1) & 0x04040404u) | 0x03020100u;
+            sel_o = ((so >> 1) & 0x04040404u) | 0x03020100u;
+        }
     }
     const uint32_t le = plane_lookup4<B>(lo, se, se7, sel_e), he = plane_lookup4<B>(hi, se, se7, sel_e);
     const uint32_t lo_ = plane_lookup4<B>(lo, so, so7, sel_o), ho = plane_lookup4<B>(hi, so, so7, sel_o);

@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * kWaves, 4) void stream_kernel(StreamArgs A) {
                        }
 #pragma unroll
                        for (int j = 0; j < 4; ++j)
-                           mma(s, j, __builtin_bit_cast(bf16x8_t, regtab_lookup8_eo<B>(lo, hi, Wt::template code<!kNested>(st, j))));
+                           mma(s, j, __builtin_bit_cast(bf16x8_t, regtab_lookup8_eo<B, true>(lo, hi, Wt::template code<!kNested>(st, j))));
                    });
         };
         if constexpr (kNested) {
