@@ -472,8 +472,9 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
         gemv = false;
     }
 
-    // few positions per expert: the projections of stream.hip
-    const int stream_n = gemv || force_path == 0 ? stream_positions(d, T, ke, gemv) : 0;
+    // few positions per expert: the projections of stream.hip (a forced path
+    // takes the kernels it names)
+    const int stream_n = force_path == 0 ? stream_positions(d, T, ke, gemv) : 0;
 
     char* ws = (char*)workspace;
     uint16_t* act = (uint16_t*)(ws + L.act);

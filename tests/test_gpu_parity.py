@@ -1565,6 +1565,34 @@ def test_moe_layer_paths_agree(gpu):
     assert rel_maxabs(a, b) <= TOL
 
 
+@pytest.mark.parametrize("fmt", ["bl4", "ref", "nested"])
+def test_moe_layer_forced_paths_take_their_own_kernels(gpu, fmt):
+    """20 tokens, 5 positions an expert: auto takes the weight-streaming kernels, path 1 the
+    GEMV kernels, path 2 the grouped GEMM.  Each is right, and each adds its fp32 products in
+    another order, so no two of the three results share their bits."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    E, k, H, I, T = 8, 2, 512, 320, 20
+    if fmt == "nested":
+        bits = [2, 3, 4, 2, 3, 4, 3, 2]
+        w13, w2 = (NestedExpertset(bits, m, c, seed=s, n_iter=4) for m, c, s in ((2 * I, H, 60), (H, I, 61)))
+    else:
+        w13, w2 = _moe_case(fmt, E, 0, H, I, seed=60)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 0)
+    rng = np.random.default_rng(60)
+    xb = _x(rng, T, H)
+    rw, rids = O.route(rng.standard_normal((T, E)).astype(np.float32), k)
+    args = (moe, to_dev_bf16(xb, gpu), torch.from_numpy(rw).to(gpu), torch.from_numpy(rids).to(gpu))
+    ref = O.moe_layer(xb, rids, rw, w13.deq_f32, w2.deq_f32)
+    outs = [ops.moe_forward(*args, out_dtype=torch.float32, path=p) for p in (0, 1, 2)]
+    for out in outs:
+        assert rel_maxabs(out.cpu().numpy(), ref) <= TOL
+    assert not torch.equal(outs[0], outs[1])
+    assert not torch.equal(outs[0], outs[2])
+    assert not torch.equal(outs[1], outs[2])
+
+
 # ------------------------------------------------ dense bf16 shared expert
 
 def dense_shared_weights(gpu, Is, H, seed):
