@@ -317,6 +317,7 @@ struct RefRows {
     const uint16_t* absmax;
     void* y;
     int M, K, T, nb, bs, bs_shift, y_dtype;   // bs_shift: log2(bs), -1 if bs is no power of two
+    uint32_t at;            // weights before row 0's first in idx and in absmax's first block (M K + at < 2^32)
 };
 
 __device__ __forceinline__ uint32_t ref_block(const RefRows& a, uint32_t flat) {
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(256) void ref_gemv_rows_kernel(RefRows a) {
         cbv[i] = a.cbf ? a.cbf[4 * lane + i] : bf16_to_f32(a.cbh[4 * lane + i]);
     uint32_t flat0[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) flat0[r] = (uint32_t)min(row0 + r, a.M - 1) * (uint32_t)a.K;
+    for (int r = 0; r < R; ++r) flat0[r] = (uint32_t)min(row0 + r, a.M - 1) * (uint32_t)a.K + a.at;
     const float* cb = s_cb[wv];
     const int nwhole = a.K / kC;   // lane pieces of kC columns
     const int nb1 = a.nb - 1;
@@ -458,7 +459,7 @@ __global__ __launch_bounds__(256) void ref_gemv_generic_kernel(RefRows a) {
     for (int t = 0; t < a.T; ++t) {
         float acc = 0.f;
         for (int c = lane; c < a.K; c += 64) {
-            const uint32_t flat = (uint32_t)row * (uint32_t)a.K + (uint32_t)c;
+            const uint32_t flat = (uint32_t)row * (uint32_t)a.K + a.at + (uint32_t)c;
             const float xv = bf16_to_f32(a.x[(int64_t)t * a.K + c]);
             const float cv = s_cb[a.idx[flat]], av = bf16_to_f32(a.absmax[min((int)ref_block(a, flat), a.nb - 1)]);
             acc += kDeq ? xv * bf16_to_f32(f32_to_bf16(cv * av)) : xv * cv * av;
@@ -490,7 +491,7 @@ static void ref_gemv_rows_launch(const RefRows& a, hipStream_t s) {
 
 template <bool kDeq>
 static int ref_gemv_dispatch(const RefRows& a, hipStream_t s) {
-    const bool aligned = a.K % 16 == 0 && a.bs % 16 == 0 && (uintptr_t)a.idx % 16 == 0 && (uintptr_t)a.x % 16 == 0;
+    const bool aligned = a.K % 16 == 0 && a.bs % 16 == 0 && ((uintptr_t)a.idx + a.at) % 16 == 0 && (uintptr_t)a.x % 16 == 0;
     if (aligned) ref_gemv_rows_launch<2, kDeq, true>(a, s);
     else if (a.bs >= 8) ref_gemv_rows_launch<2, kDeq, false>(a, s);
     else hipLaunchKernelGGL(ref_gemv_generic_kernel<kDeq>, dim3((a.M + 3) / 4), dim3(256), 0, s, a);
@@ -501,8 +502,24 @@ int launch_ref_gemv(const uint16_t* x, const uint8_t* idx, const uint16_t* cb_bf
                     const float* cb_f32, const uint16_t* absmax, void* y, int M, int K, int T,
                     int num_blocks, int block_size, int y_dtype, hipStream_t s, bool dequant) {
     const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
-    const RefRows a{x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, shift, y_dtype};
-    return dequant ? ref_gemv_dispatch<true>(a, s) : ref_gemv_dispatch<false>(a, s);
+    RefRows a{x, idx, cb_bf16, cb_f32, absmax, y, M, K, T, num_blocks, block_size, shift, y_dtype, 0};
+    // The kernels count weights in 32 bits.  A larger matrix goes in ranges of
+    // rows (the entry points with several vectors take fewer than 2^31 weights)
+    const int64_t most = ((int64_t)1 << 32) - 1;
+    if ((int64_t)M * K <= most) return dequant ? ref_gemv_dispatch<true>(a, s) : ref_gemv_dispatch<false>(a, s);
+    if (T != 1) return LUTMOE_EUNSUPPORTED;
+    const int64_t rows = (most - (block_size - 1)) / K;   // at least one: K, block_size < 2^31
+    for (int64_t r0 = 0; r0 < M; r0 += rows) {
+        const int64_t first = r0 * K, b0 = first / block_size < num_blocks ? first / block_size : num_blocks - 1;
+        a.at = (uint32_t)(first % block_size);
+        a.idx = idx + first - a.at;
+        a.absmax = absmax + b0;   // (past the last block: that one for every weight)
+        a.nb = num_blocks - (int)b0;
+        a.M = (int)(M - r0 < rows ? M - r0 : rows);
+        a.y = (char*)y + r0 * (y_dtype == LUTMOE_DTYPE_F32 ? 4 : 2);
+        if (const int rc = dequant ? ref_gemv_dispatch<true>(a, s) : ref_gemv_dispatch<false>(a, s)) return rc;
+    }
+    return LUTMOE_OK;
 }
 
 template <class Dec, bool kXF32>

@@ -367,6 +367,34 @@ def test_lut_gemv_reference_signature(gpu):
     assert rel_maxabs(O.bf16_to_f32(bf16_bits(out)), ref) <= TOL + 2.0 ** -8
 
 
+@pytest.mark.parametrize("K", [65536, 65521])
+def test_lut_gemv_reference_signature_past_4gb(gpu, K):
+    """launch_lut_gemv_kernel has no limit on M * K: rows past the 2^32nd weight take their own
+    codes and absmax (whole and odd rows)."""
+    import torch
+    from block_lut_amd import _native as N
+    M = 2 ** 32 // K + 9
+    nb = -(-M * K // 128)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    idx = torch.randint(0, 256, (M, K), dtype=torch.uint8, generator=g, device=gpu)
+    am = (torch.rand(nb, generator=g, device=gpu) * 0.02 + 0.01).to(torch.bfloat16)
+    x = torch.randn(K, generator=g, device=gpu).to(torch.bfloat16)
+    cb = torch.from_numpy(O.bf16_to_f32(golden_codebook())).to(gpu)
+    out = torch.empty(M, dtype=torch.bfloat16, device=gpu)
+    torch.cuda.synchronize()
+    N.lib().launch_lut_gemv_kernel(x.data_ptr(), idx.data_ptr(), cb.data_ptr(), am.data_ptr(),
+                                   out.data_ptr(), M, K, nb)
+    N.check_last("launch_lut_gemv_kernel")
+    torch.cuda.synchronize()
+    for row in (0, 1, 2 ** 31 // K, 2 ** 32 // K - 1, 2 ** 32 // K, 2 ** 32 // K + 1, M - 1):
+        block = (torch.arange(K, device=gpu) + row * K) // 128
+        w = cb.double()[idx[row].long()] * am.double()[block]
+        p = w * x.double()
+        ref, terms = p.sum(), p.abs().sum()
+        # the bf16 rounding of the result, and K fp32 roundings of at most the sum of magnitudes
+        assert (out[row].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + (K + 4) * 2.0 ** -24 * terms
+
+
 # ------------------------------------------------------------------ routing
 
 @pytest.mark.parametrize("T,E,k,renorm", [(1, 60, 4, False), (37, 64, 6, False), (513, 8, 2, True)])
