@@ -241,6 +241,17 @@ def new_workspace(moe: MoEWeights, T: int, k: int, device) -> torch.Tensor:
     return torch.zeros(max(moe_workspace_bytes(moe, T, k), 256), dtype=torch.uint8, device=device)
 
 
+def _scratch(moe: MoEWeights, T: int, k: int, stages: int, device, workspace: Optional[torch.Tensor]) -> torch.Tensor:
+    """The caller's workspace, or one for this call where that is missing or too small.  A call
+    of some stages alone reads routing that it does not write: zeros (no pair, no work) where
+    no earlier call can have left any."""
+    need = max(moe_workspace_bytes(moe, T, k), 256)
+    if workspace is not None and workspace.numel() >= need:
+        return workspace
+    new = torch.empty if stages == N.STAGE_ALL else torch.zeros
+    return new(need, dtype=torch.uint8, device=device)
+
+
 def moe_forward(moe: MoEWeights, x: torch.Tensor, topk_weights: torch.Tensor,
                 topk_ids: torch.Tensor, out: Optional[torch.Tensor] = None,
                 out_dtype: torch.dtype = torch.bfloat16, path: int = PATH_AUTO,
@@ -260,9 +271,7 @@ def moe_forward(moe: MoEWeights, x: torch.Tensor, topk_weights: torch.Tensor,
     else:
         _dev(out, out.dtype, "out")
         out_dtype = out.dtype
-    need = moe_workspace_bytes(moe, T, k)
-    if workspace is None or workspace.numel() < need:
-        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)   # (needs no zeroing)
+    workspace = _scratch(moe, T, k, stages, x.device, workspace)
     d = moe.desc()
     N.check("lutmoe_moe_forward",
             N.lib().lutmoe_moe_forward_stages(ctypes.byref(d), x.data_ptr(), w.data_ptr(),
@@ -295,9 +304,7 @@ def moe_forward_logits(moe: MoEWeights, x: torch.Tensor, logits: torch.Tensor, t
     else:
         _dev(out, out.dtype, "out")
         out_dtype = out.dtype
-    need = moe_workspace_bytes(moe, T, top_k)
-    if workspace is None or workspace.numel() < need:
-        workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)   # (needs no zeroing)
+    workspace = _scratch(moe, T, top_k, stages, x.device, workspace)
     d = moe.desc()
     flags = ((N.ROUTE_RENORM if renormalize else 0) | (N.ROUTE_BF16_WEIGHTS if bf16_weights else 0) |
              (N.ROUTE_BF16_LOGITS if lg16 else 0))

@@ -156,3 +156,55 @@ def test_fused_lut_moe_op_fake_shapes():
         assert tuple(out.shape) == (T, H) and out.dtype == torch.bfloat16
         out1 = torch.ops.lutmoe.fused_lut_moe(x[0], ids[:1], w[:1], w13, a13, w2, a2, cb)
         assert tuple(out1.shape) == (1, H)
+
+
+class _RecordingLib:
+    """Stands in for the C library: keeps a copy of the workspace each layer call is given."""
+
+    def __init__(self):
+        self.seen = []
+
+    def lutmoe_moe_workspace_size(self, d, T, k):
+        return 4096
+
+    def _call(self, ws, n):
+        import ctypes
+        self.seen.append(bytes((ctypes.c_uint8 * n).from_address(ws)))
+        return 0
+
+    def lutmoe_moe_forward_stages(self, d, x, w, ids, T, k, out, dt, ws, n, path, stages, stream):
+        return self._call(ws, n)
+
+    def lutmoe_moe_forward_logits_ex(self, d, x, lg, T, k, flags, scaling, out, dt, ws, n, path, stages, stream):
+        return self._call(ws, n)
+
+
+@pytest.mark.parametrize("entry", ["ids", "logits"])
+def test_scratch_of_partial_stages_is_zeroed(monkeypatch, entry):
+    """A call of some stages alone, without a workspace that an earlier call filled, finds
+    zeros where it reads the routing (no pairs): memory as the allocator hands it out would
+    be taken for row and expert numbers."""
+    import types
+    from block_lut_amd import ops
+    lib = _RecordingLib()
+    monkeypatch.setattr(ops.N, "lib", lambda: lib)
+    monkeypatch.setattr(ops, "_dev", lambda t, dtype, name: t)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops.ctypes, "byref", lambda d: d)
+    T, k, H, E = 3, 2, 64, 4
+    moe = types.SimpleNamespace(hidden=H, num_routed=E, desc=lambda: None)
+    x = torch.zeros(T, H, dtype=torch.bfloat16)
+    det = torch.are_deterministic_algorithms_enabled()
+    torch.use_deterministic_algorithms(True)      # (torch.empty fills its memory with ones)
+    try:
+        assert torch.empty(16, dtype=torch.uint8).eq(255).all()
+        for stages in (ops.N.STAGE_GATE_UP, ops.N.STAGE_DOWN, ops.N.STAGE_GATE_UP | ops.N.STAGE_DOWN):
+            for ws in (None, torch.full((4095,), 255, dtype=torch.uint8)):
+                if entry == "ids":
+                    ops.moe_forward(moe, x, torch.zeros(T, k), torch.zeros(T, k, dtype=torch.int32),
+                                    workspace=ws, stages=stages)
+                else:
+                    ops.moe_forward_logits(moe, x, torch.zeros(T, E), k, workspace=ws, stages=stages)
+                assert len(lib.seen[-1]) == 4096 and not any(lib.seen[-1])
+    finally:
+        torch.use_deterministic_algorithms(det)
