@@ -103,7 +103,10 @@ class LUTMoELayer(nn.Module):
         shape = hidden_states.shape
         x = hidden_states.reshape(-1, shape[-1])
         xb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16)).contiguous()
-        logits = self._logits(xb)
+        # the logits in the dtype they are computed in, unless a subclass or a caller has
+        # replaced router_logits
+        own = getattr(self.router_logits, "__func__", None) is _ROUTER_LOGITS
+        logits = self._logits(xb) if own else self.router_logits(xb)
         need = ops.moe_workspace_bytes(self.moe, xb.shape[0], self.top_k)
         if self._ws is None or self._ws.numel() < need or self._ws.device != xb.device:
             self._ws = ops.new_workspace(self.moe, xb.shape[0], self.top_k, xb.device)
@@ -120,3 +123,6 @@ class LUTMoELayer(nn.Module):
                                     scaling=self.routed_scaling_factor)
             out = ops.moe_forward(self.moe, xb, w.to(torch.bfloat16).float(), ids, workspace=self._ws)
         return out.to(hidden_states.dtype).reshape(shape)
+
+
+_ROUTER_LOGITS = LUTMoELayer.router_logits

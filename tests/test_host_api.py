@@ -208,3 +208,33 @@ def test_scratch_of_partial_stages_is_zeroed(monkeypatch, entry):
                 assert len(lib.seen[-1]) == 4096 and not any(lib.seen[-1])
     finally:
         torch.use_deterministic_algorithms(det)
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+@pytest.mark.parametrize("router_dtype", [torch.bfloat16, torch.float32])
+def test_layer_routes_by_a_replaced_router_logits(monkeypatch, how, router_dtype):
+    """LUTMoELayer.forward routes by router_logits, also where a subclass, an instance or a
+    patch of the class replaces it."""
+    import types
+    from block_lut_amd import moe_layer
+    from block_lut_amd.moe_layer import LUTMoELayer
+    E, H, k, T = 8, 64, 2, 3
+    seen = []
+    monkeypatch.setattr(moe_layer.ops, "moe_workspace_bytes", lambda moe, T, k: 256)
+    monkeypatch.setattr(moe_layer.ops, "new_workspace", lambda moe, T, k, dev: torch.zeros(256, dtype=torch.uint8))
+    monkeypatch.setattr(moe_layer.ops, "router_logits", lambda x, gate, round_bf16: torch.zeros(x.shape[0], E))
+    monkeypatch.setattr(moe_layer.ops, "moe_forward_logits",
+                        lambda moe, x, logits, top_k, **kw: seen.append(logits) or torch.zeros_like(x))
+    mine = torch.arange(T * E, dtype=torch.float32).view(T, E)
+
+    class Mine(LUTMoELayer):
+        def router_logits(self, xb):
+            return mine
+    moe = types.SimpleNamespace(num_routed=E, hidden=H)
+    layer = (Mine if how == "subclass" else LUTMoELayer)(moe, torch.zeros(E, H), k, router_dtype=router_dtype)
+    if how == "instance":
+        layer.router_logits = lambda xb: mine
+    elif how == "class":
+        monkeypatch.setattr(LUTMoELayer, "router_logits", lambda self, xb: mine)
+    layer(torch.zeros(T, H))
+    assert seen[0] is mine
