@@ -181,10 +181,16 @@ __device__ void cta_route(const DecodeArgs& A, RouteOut& R, RouteScratch& X) {
                     R.pw[t * ke + lane] = routed_weight(pj, wsum, A.renorm, A.scaling);
                 }
             } else {
+                // (NaN never selected; slots past the last number: dropped, weight 0)
+                if (lane < k) {
+                    X.pid[t * ke + lane] = -1;
+                    R.pw[t * ke + lane] = 0.f;
+                }
+                wave_lds_sync();
                 float lsum = 0.f;
                 for (int e = lane; e < E; e += 64) {
                     const float v = src[e];
-                    int r = 0;
+                    int r = v != v ? k : 0;
 #pragma unroll 8
                     for (int q = 0; q < E; ++q) {
                         const float u = src[q];

@@ -936,6 +936,35 @@ def test_moe_layer_from_logits_ties(gpu, T, E, renorm):
     assert rel_maxabs(out.cpu().numpy(), ref) <= TOL
 
 
+@pytest.mark.parametrize("T", [1, 2, 4])
+@pytest.mark.parametrize("E", [60, 130])
+def test_moe_layer_from_logits_nan(gpu, T, E):
+    """Decode routing on logits with NaN (one and several logits a lane): NaN is never selected
+    and a slot with only NaN left is dropped, as in the top-k kernel, so the layer from logits
+    is the layer from that kernel's ids and weights."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    S, k, H, I = 1, 4, 256, 192
+    w13, w2 = _moe_case("bl4", E, S, H, I, seed=95)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, S)
+    rng = np.random.default_rng(950 + T + E)
+    x = to_dev_bf16(_x(rng, T, H), gpu)
+    lg = rng.standard_normal((T, E)).astype(np.float32)
+    lg[0, :] = np.nan                        # no expert at all: the shared one alone
+    if T > 1:
+        lg[1, 2:] = np.nan                   # two numbers left for four slots
+    if T > 2:
+        lg[2, ::7] = np.nan
+    logits = torch.from_numpy(lg).to(gpu)
+    out = ops.moe_forward_logits(moe, x, logits, k, out_dtype=torch.float32)
+    w, ids = ops.route_topk(logits, k)
+    ref = ops.moe_forward(moe, x, w, ids, out_dtype=torch.float32)
+    assert (ids[0] == -1).all() and not out[0].isnan().any()
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert rel_maxabs(out.nan_to_num().cpu().numpy(), ref.nan_to_num().cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("fmt,T", [("bl4", 1), ("bl4", 2), ("bl4", 9), ("ref", 1), ("nested", 1)])
 def test_moe_layer_decode_staged_equals_full(gpu, fmt, T):
     """The decode layer run stage by stage (routing + gate/up, then down + combine, in one
