@@ -479,6 +479,19 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     char* ws = (char*)workspace;
     uint16_t* act = (uint16_t*)(ws + L.act);
     hipStream_t s = stream_of(stream);
+    // Weights rounded to bf16 come from the top-k kernel where the routing inside
+    // the decode kernels adds the softmax up in another order (several logits a
+    // lane): a last bit there would move a weight by a bf16 step
+    if (gemv && by_logits && (flags & LUTMOE_ROUTE_BF16_WEIGHTS) && d->num_routed > 64) {
+        float* tw = (float*)(ws + L.topk_w);
+        int32_t* ti = (int32_t*)(ws + L.topk_ids);
+        if ((stages & LUTMOE_STAGE_ROUTE) &&
+            (rc = launch_route_topk(logits, false, T, d->num_routed, k, renorm, scaling, tw, ti, s)))
+            return rc;
+        topk_w = tw;
+        topk_ids = ti;
+        logits = nullptr;
+    }
     // the dense shared expert: gate/up with the gate/up stage, its weighted
     // rows with the down stage, before the kernels that write the output
     // (which add them)

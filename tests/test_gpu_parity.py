@@ -1744,8 +1744,7 @@ def test_dense_shared_expert_shapes(gpu, T, H, Is):
 def test_forward_logits_bf16_router(gpu, T, E, renorm):
     """A bf16 router's routing inside the layer call (weights rounded to bf16; past 64 tokens
     the logits read as bf16) against the top-k kernel, the cast and the layer from ids, with
-    ties between the bf16 logits.  E <= 64: the same bits; above, the softmax sums in another
-    order, so a weight may round to its neighbour (2^-8 of it)."""
+    ties between the bf16 logits: the same bits."""
     import torch
     from block_lut_amd import ops
     from block_lut_amd.formats import MoEWeights
@@ -1759,10 +1758,35 @@ def test_forward_logits_bf16_router(gpu, T, E, renorm):
                                  bf16_weights=True)
     w, ids = ops.route_topk(lg, k, renormalize=renorm, scaling=1.5)
     ref = ops.moe_forward(moe, x, w.to(torch.bfloat16).float(), ids, out_dtype=torch.float32)
-    if E <= 64:
+    assert torch.equal(out, ref)
+    unrounded = ops.moe_forward(moe, x, w, ids, out_dtype=torch.float32)
+    assert not torch.equal(out, unrounded)
+
+
+@pytest.mark.parametrize("T,E", [(1, 130), (2, 60), (2, 130), (20, 60), (20, 130), (20, 320)])
+def test_forward_logits_bf16_router_at_rounding_boundaries(gpu, T, E):
+    """Scalings that put one routed weight on the middle between two bf16 numbers: the weight
+    the layer call rounds has the top-k kernel's last bit, so both round the same way."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    k, H, I = 4, 64, 64
+    w13, w2 = _moe_case("bl4", 1, 0, H, I, seed=33)      # (E experts of the same codes)
+
+    def stack(w):
+        one = w.stack(gpu)
+        return type(one)(one.codes.repeat(E, 1, 1).contiguous(), one.tables.repeat(E, 1, 1, 1).contiguous())
+    moe = MoEWeights(stack(w13), stack(w2), H, I, E, 0)
+    rng = np.random.default_rng(33 + T)
+    x = to_dev_bf16(_x(rng, T, H), gpu)
+    lg = torch.from_numpy(rng.standard_normal((T, E)).astype(np.float32)).to(gpu).to(torch.bfloat16)
+    p = ops.route_topk(lg, k)[0].flatten().cpu().numpy()
+    for i in range(0, 24):
+        scale = float(np.float32(1 + 2.0 ** -8) / p[i % p.size]) * (1 + (i // p.size) * 2.0 ** -7)
+        w, ids = ops.route_topk(lg, k, scaling=scale)
+        ref = ops.moe_forward(moe, x, w.to(torch.bfloat16).float(), ids, out_dtype=torch.float32)
+        out = ops.moe_forward_logits(moe, x, lg, k, scaling=scale, out_dtype=torch.float32, bf16_weights=True)
         assert torch.equal(out, ref)
-    else:
-        assert rel_maxabs(out.cpu().numpy(), ref.cpu().numpy()) <= 2.0 ** -8
 
 
 @pytest.mark.parametrize("fmt", ["bl4", "ref", "nested"])
