@@ -77,8 +77,11 @@ int validate_ref_vector(const lutmoe_weights* w) {
 size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct MoeLayout {
-    size_t route, topk_w, topk_ids, pair_ids, pair_w, offsets, perm, inv, active, sched, act, y, dact, dy, dw, total;
-    int dy_splits;   // K splits of the dense down projection that fit
+    size_t route, topk_w, topk_ids, pair_ids, pair_w, offsets, perm, inv, active, sched, act, y, dact, dy, dw;
+    size_t least, total;   // bytes a call needs, and those it makes use of
+    size_t dy_row;         // bytes of one result of the dense down projection
+    // K splits of the dense down projection that fit in a workspace
+    int dy_splits(size_t bytes) const { return dy_row ? (int)(((bytes < total ? bytes : total) - dy) / dy_row) : 1; }
 };
 
 // Room for two K-split partial results of the down projection when that is
@@ -111,14 +114,14 @@ MoeLayout moe_layout(const lutmoe_moe_desc* d, int T, int k) {
     // fixed scratch of lutmoe_moe_forward_noalloc only with them stays within
     // it (so the size still grows with T)
     L.dy = o;
-    const size_t row = (size_t)d->hidden * 4, one = (size_t)T * row;
+    const size_t row = (size_t)d->hidden * 4;
+    L.dy_row = Is ? (size_t)T * row : 0;
     size_t rows = (size_t)T * 8 < 2048 ? (size_t)T * 8 : 2048;
     if (rows < (size_t)T) rows = T;
-    const size_t base = align_up(o + (Is ? one : 0));
+    L.least = align_up(o + L.dy_row);
     size_t with = align_up(o + (Is ? rows * row : 0));
     if (with > kNoallocScratch) with = kNoallocScratch;
-    L.total = base > with ? base : with;
-    L.dy_splits = one ? (int)((L.total - o) / one) : 1;
+    L.total = L.least > with ? L.least : with;
     return L;
 }
 
@@ -457,7 +460,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     if (logits_bf16 && T <= 64) return LUTMOE_EUNSUPPORTED;
     if (!aligned(x, 16) || !aligned(out, 16) || !aligned(workspace, 256)) return LUTMOE_EALIGN;
     const MoeLayout L = moe_layout(d, T, k);
-    if (ws_bytes < L.total) return LUTMOE_EWORKSPACE;
+    if (ws_bytes < L.least) return LUTMOE_EWORKSPACE;
     const int S = d->num_shared, E = d->num_routed, E_tot = E + S, ke = k + S;
     const int64_t P = (int64_t)T * ke;
     if (P >= (1ll << 31) / (d->hidden > d->inter ? d->hidden : d->inter)) return LUTMOE_EUNSUPPORTED;
@@ -503,7 +506,7 @@ int moe_forward_impl(const lutmoe_moe_desc* d, const void* x, const float* topk_
     int naddend = 1;   // (the decode kernels add one array)
     if (dense && (stages & LUTMOE_STAGE_DOWN) &&
         (rc = launch_dense_down(d, (const uint16_t*)(ws + L.dact), T, (const float*)(ws + L.dw),
-                                (float*)(ws + L.dy), gemv ? 1 : L.dy_splits, &naddend, s)))
+                                (float*)(ws + L.dy), gemv ? 1 : L.dy_splits(ws_bytes), &naddend, s)))
         return rc;
     if (gemv) {
         // routing + permutation happen inside both decode kernels

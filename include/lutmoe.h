@@ -257,7 +257,9 @@ int lutmoe_permute(const int32_t* topk_ids_dev, int T, int k, int E, int32_t* of
 
 /* ---- fused MoE layer ------------------------------------------------------ */
 
-/* Workspace bytes lutmoe_moe_forward needs for T tokens and top-k.
+/* Workspace bytes lutmoe_moe_forward makes use of for T tokens and top-k.  (With
+ * a dense shared expert that includes room for K splits of its down projection;
+ * a workspace with less of it, down to one result of T rows, is taken too.)
  * The workspace is device memory, 256-byte aligned, owned by the caller; its
  * contents need no initialisation (every kernel writes what it reads within
  * the call).  Calls that overlap in time must not share a workspace. */

@@ -1739,6 +1739,43 @@ def test_dense_shared_expert_shapes(gpu, T, H, Is):
     assert ((out - ref).norm() / ref.norm()) < 1e-3
 
 
+@pytest.mark.parametrize("T,Is", [(5, 640), (65, 2048), (129, 1088)])
+def test_dense_shared_expert_least_workspace(gpu, T, Is):
+    """A workspace with room for one result of the dense down projection and none for its K
+    splits (the layer's without the dense expert, the expert's activations, token weights and
+    one result) is taken; one byte less is refused; nothing is written past it."""
+    import ctypes
+    import torch
+    from block_lut_amd import _native as N
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    E, k, H, I = 4, 2, 192, 64
+    w13, w2 = _moe_case("bl4", E, 0, H, I, seed=19)
+    d13, d2, _, _ = dense_shared_weights(gpu, Is, H, T)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 0, dense_shared=(d13, d2))
+    rng = np.random.default_rng(T)
+    x = to_dev_bf16(_x(rng, T, H), gpu)
+    w, ids = ops.route_topk(torch.from_numpy(rng.standard_normal((T, E)).astype(np.float32)).to(gpu), k)
+    full = ops.moe_forward(moe, x, w, ids, out_dtype=torch.float32)
+
+    def up(v):
+        return (v + 255) // 256 * 256
+    least = ops.moe_workspace_bytes(MoEWeights(moe.w13, moe.w2, H, I, E, 0), T, k)
+    least = up(up(up(least + T * Is * 2) + T * 4) + T * H * 4)
+    assert least < ops.moe_workspace_bytes(moe, T, k)
+    ws = torch.full((least + 4096,), 0xAB, dtype=torch.uint8, device=gpu)
+    out = torch.empty((T, H), device=gpu)
+
+    def call(n):
+        return N.lib().lutmoe_moe_forward(ctypes.byref(moe.desc()), x.data_ptr(), w.data_ptr(), ids.data_ptr(), T, k,
+                                          out.data_ptr(), N.DTYPE_F32, ws.data_ptr(), n, 0,
+                                          torch.cuda.current_stream().cuda_stream)
+    assert call(least - 1) == N.LUTMOE_EWORKSPACE
+    assert call(least) == N.LUTMOE_OK
+    assert (ws[least:] == 0xAB).all()
+    assert rel_maxabs(out.cpu().numpy(), full.cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 33, 65])
 @pytest.mark.parametrize("E,renorm", [(12, False), (60, True), (130, False)])
 def test_forward_logits_bf16_router(gpu, T, E, renorm):
