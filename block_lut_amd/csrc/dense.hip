@@ -445,7 +445,9 @@ inline int dense_row_blocks(bool gate_up, int H, int I) {
 struct DenseTiles {
     int nmw, ns;
 };
-inline DenseTiles dense_tiles(int T, int nxb, int max_split, int nk) {
+inline DenseTiles dense_tiles(bool gate_up, int T, int H, int I, int max_split) {
+    if (T <= kSkMaxT) return DenseTiles{0, 1};   // (dense_skinny_kernel)
+    const int nxb = dense_row_blocks(gate_up, H, I), nk = (gate_up ? H : I) / kDBK;
     const int cu = lutmoe_host::cu_count(), ncu = cu > 0 ? cu : 256;
     DenseTiles best{1, 1};
     float best_cost = 0.f;
@@ -480,8 +482,8 @@ int dense_gemv_launch(const uint16_t* W, int M, int K, int I, const uint16_t* x,
 
 template <bool kGateUp>
 int dense_mfma_launch(const uint16_t* W, const uint16_t* src, int T, int H, int I, const float* tokw, void* dst,
-                      int ns, const TokenWeights& tw, hipStream_t s) {
-    if (T <= kSkMaxT) {
+                      const DenseTiles& tiles, const TokenWeights& tw, hipStream_t s) {
+    if (!tiles.nmw) {
         const dim3 grid((kGateUp ? I : H) / 16 + (kGateUp ? 1 : 0)), block(64 * kSkWaves);
         if (T <= 16)
             hipLaunchKernelGGL((dense_skinny_kernel<kGateUp, 1>), grid, block, 0, s, W, src, T, H, I, tokw, dst, tw);
@@ -490,7 +492,6 @@ int dense_mfma_launch(const uint16_t* W, const uint16_t* src, int T, int H, int 
         return lutmoe_host::check_launch();
     }
     const int nxb = dense_row_blocks(kGateUp, H, I);
-    const DenseTiles tiles = dense_tiles(T, nxb, kGateUp ? 1 : ns, (kGateUp ? H : I) / kDBK);
     const int64_t stride = (int64_t)T * H;
 #define LUTMOE_DENSE_TILE(NMW)                                                                                      \
     hipLaunchKernelGGL((dense_tile_kernel<kGateUp, NMW>),                                                           \
@@ -517,7 +518,7 @@ int launch_dense_gate_up(const lutmoe_moe_desc* d, const uint16_t* x, int T, uin
     const uint16_t* W = (const uint16_t*)d->dense_w13;
     const TokenWeights tw{(const uint16_t*)d->shared_gate, tokw};
     if (T <= 4) return dense_gemv_launch<true>(W, 2 * I, H, I, x, T, nullptr, act, tw, s);
-    return dense_mfma_launch<true>(W, x, T, H, I, nullptr, act, 1, tw, s);
+    return dense_mfma_launch<true>(W, x, T, H, I, nullptr, act, dense_tiles(true, T, H, I, 1), tw, s);
 }
 
 int launch_dense_down(const lutmoe_moe_desc* d, const uint16_t* act, int T, const float* tokw, float* y,
@@ -526,8 +527,9 @@ int launch_dense_down(const lutmoe_moe_desc* d, const uint16_t* act, int T, cons
     const uint16_t* W = (const uint16_t*)d->dense_w2;
     *nsplit = 1;
     if (T <= 4) return dense_gemv_launch<false>(W, H, I, I, act, T, tokw, y, TokenWeights{}, s);
-    if (T > kSkMaxT) *nsplit = dense_tiles(T, dense_row_blocks(false, H, I), max_split, I / kDBK).ns;
-    return dense_mfma_launch<false>(W, act, T, H, I, tokw, y, *nsplit, TokenWeights{}, s);
+    const DenseTiles tiles = dense_tiles(false, T, H, I, max_split);
+    *nsplit = tiles.ns;
+    return dense_mfma_launch<false>(W, act, T, H, I, tokw, y, tiles, TokenWeights{}, s);
 }
 
 }  // namespace lutmoe_host
