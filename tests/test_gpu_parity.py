@@ -1834,8 +1834,8 @@ def test_moe_layer_few_positions_per_expert(gpu, fmt, T, E, k, H, I, skew):
     """The weight-streaming projections (stream.hip) at their edges, the layer against the
     oracle: items of 16 and 32 positions, full, left over and cut from one heavy expert
     (skew), dropped pairs, K of one and more 128-column steps with a last one of 64, more
-    columns than LDS holds of the activations, a K long enough for its two splits, half a
-    CTA's rows; decode and prefill routing."""
+    columns than LDS holds of the activations, half a CTA's rows; decode and prefill
+    routing."""
     import torch
     from block_lut_amd import ops
     from block_lut_amd.formats import MoEWeights
@@ -1861,3 +1861,31 @@ def test_moe_layer_few_positions_per_expert(gpu, fmt, T, E, k, H, I, skew):
     ref = O.moe_layer(xb, np.where(keep, rids, 0), np.where(keep, rw, 0), w13.deq_f32, w2.deq_f32,
                       shared=[(w13.deq_f32(E), w2.deq_f32(E))])
     assert rel_maxabs(out, ref) <= TOL
+
+
+@pytest.mark.parametrize("fmt", ["bl4", "ref", "nested"])
+@pytest.mark.parametrize("T,I", [(12, 4160), (40, 4096), (40, 4160)])
+def test_moe_layer_few_positions_down_split(gpu, fmt, T, I):
+    """The weight-streaming down projection split over K (I >= 4096 columns on few CTAs), the
+    last step of its second half with 128 and with 64 columns, decode and prefill: both
+    halves' results are written, and the layer is the oracle's."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    E, k, H = 3, 2, 128
+    if fmt == "nested":
+        w13, w2 = (NestedExpertset([2, 3, 4], m, c, seed=s, n_iter=2) for m, c, s in ((2 * I, H, 710), (H, I, 711)))
+    else:
+        w13, w2 = _moe_case(fmt, E, 0, H, I, seed=710)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 0)
+    rng = np.random.default_rng(T + I)
+    xb = _x(rng, T, H)
+    rw, rids = O.route(rng.standard_normal((T, E)).astype(np.float32), k)
+    ws = ops.new_workspace(moe, T, k, gpu).fill_(0xFF)
+    out = ops.moe_forward(moe, to_dev_bf16(xb, gpu), torch.from_numpy(rw).to(gpu), torch.from_numpy(rids).to(gpu),
+                          out_dtype=torch.float32, workspace=ws).cpu().numpy()
+    # the results of the two halves [2][T k][H] fp32 end the workspace
+    halves = ws[ws.numel() - 2 * T * k * H * 4:].view(torch.float32).view(2, T * k, H)
+    assert halves.isfinite().all()
+    assert (halves[0] - halves[1]).abs().max() > 0
+    assert rel_maxabs(out, O.moe_layer(xb, rids, rw, w13.deq_f32, w2.deq_f32)) <= TOL
