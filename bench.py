@@ -77,12 +77,12 @@ def measured_traffic(name):
 def decode_kernel_label(T, P, E_tot):
     """The gate/up kernel the library launches for this batch (BL4; api.cpp's
     stream_positions and decode.hip's tb_for): one token its own kernel, the streaming MFMA
-    kernel from 1.4 to 27 positions an active expert, else two-token passes up to 16 tokens
-    (and up to 32 while the experts hold at most 3 positions on average)."""
+    kernel from 1.4 positions an active expert (past 32 tokens up to 27), else two-token passes up
+    to 16 tokens (and up to 32 while the experts hold at most 3 positions on average)."""
     if T <= 1:
         return "bl4_decode_gate_up_t1"
     experts = min(P, E_tot)
-    if T > 2 and E_tot <= 512 and 7 * experts <= 5 * P and P <= 27 * experts:
+    if T > 2 and E_tot <= 512 and 7 * experts <= 5 * P and (T <= 32 or P <= 27 * experts):
         return f"stream_kernel<gate_up, {2 if P > 10 * experts else 1}>"
     tb = 2 if T <= 16 or (T <= 32 and P <= 3 * experts) else 4
     return f"bl4_decode_gate_up<{tb}>"

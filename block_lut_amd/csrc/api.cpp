@@ -417,25 +417,34 @@ static int stream_max_chunks(int64_t P, int E_tot, int positions) {
 // Positions per work item of the stream.hip projections, 0: not taken.  By the
 // average positions of an active expert (at most; Qwen / DeepSeek / Mixtral
 // shapes and small ones, MI355X, us a layer, stream against the other path):
-//  * past about 27 an item's weights are read and looked up again for its
-//    second 32 positions, and the 256-row tiles of the ring kernels win (26.7:
-//    174 / 202, 32: 520 / 427);
+//  * more than 32 tokens: past about 27 an item's weights are read and looked up
+//    again for its second 32 positions, and the 256-row tiles of the ring kernels
+//    win (24: 416 / 406, 26.7: 174 / 202, 32: 520 / 427).  Below, also with most
+//    positions on few experts (Zipf exponents up to 1.6) or on shared slots, the
+//    items are the faster ones or within 2 % (948 layers of 33 to 400 tokens);
+//    only where every token takes the same experts do they lose (256 tokens 79 /
+//    99, 400 121 / 102), which the host does not see;
+//  * decode: an expert's positions are one item, so there is no upper limit (28
+//    and 32, 8 experts: 47 / 180 and 49 / 204 with the GEMV's four-token passes);
 //  * up to 10, items of 16 positions (of 32: 8.5 144 / 149, 17 189 / 158);
 //  * decode, BL4: the one- and two-token passes read rows in order and win
-//    while most experts hold one position (1.07: 95 / 91, 1.27: 97 / 99, 2.1:
-//    120 / 145); NestedLUT from 18 pairs (16: 26 / 24, 24: 54 / 54, 48: 65 / 72),
-//    REF from 6 (3: 37 / 32, 6: 37 / 40, 76: 108 / 143).
+//    while most experts hold one position (1.07: 91 / 87, 1.2: 97 / 95, 1.33: 95 /
+//    100, 1.6: 109 / 115; with 12 and 16 experts the lines cross near 1.7, where
+//    the stream gives up 4-8 %).  NestedLUT from 18 pairs (16: 41 / 38, 20: 47 /
+//    45, 24: 48 / 46 at 60 experts, 48 / 49 at 66, 44 / 49 at 128, 32: 56 / 56,
+//    40: 58 / 62).  REF from 6 (6: 39 / 40, 8: 39 / 41, 12: 48 / 50, 20: 55 / 63),
+//    with one slot a token from 8 (6: 39 / 33, 7: 83 / 78, 8: 39 / 40 and 87 / 92).
 static int stream_positions(const lutmoe_moe_desc* d, int T, int ke, bool gemv) {
     const int E_tot = d->num_routed + d->num_shared;
     const int64_t P = (int64_t)T * ke, experts = P < E_tot ? P : E_tot;
-    if (T <= 2 || E_tot > 512 || P > 27 * experts || !stream_supported(d)) return 0;
+    if (T <= 2 || E_tot > 512 || (!gemv && P > 27 * experts) || !stream_supported(d)) return 0;
     const int n = P > 10 * experts ? 32 : 16;
     if (stream_max_chunks(P, E_tot, n) > lutmoe::kMaxChunks) return 0;
     if (!gemv) return n;
     switch (d->w13.format) {
         case LUTMOE_FMT_BL4: return 5 * P >= 7 * experts ? n : 0;
         case LUTMOE_FMT_NESTED: return P >= 18 ? n : 0;
-        default: return P >= 6 ? n : 0;
+        default: return P >= (ke == 1 ? 8 : 6) ? n : 0;
     }
 }
 

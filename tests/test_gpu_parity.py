@@ -1889,3 +1889,29 @@ def test_moe_layer_few_positions_down_split(gpu, fmt, T, I):
     assert halves.isfinite().all()
     assert (halves[0] - halves[1]).abs().max() > 0
     assert rel_maxabs(out, O.moe_layer(xb, rids, rw, w13.deq_f32, w2.deq_f32)) <= TOL
+
+
+@pytest.mark.parametrize("fmt", ["bl4", "ref", "nested"])
+@pytest.mark.parametrize("T", [27, 28, 32])
+def test_moe_layer_every_token_on_every_expert(gpu, fmt, T):
+    """Decode with every expert on every token, at and past 27 positions an expert: one work item
+    an expert, on the streaming kernels (whose fp32 sums differ from the GEMV path's in their
+    bits)."""
+    import torch
+    from block_lut_amd import ops
+    from block_lut_amd.formats import MoEWeights
+    E, H, I = 4, 192, 128
+    if fmt == "nested":
+        w13, w2 = (NestedExpertset([2, 3, 4, 2], m, c, seed=s, n_iter=4) for m, c, s in ((2 * I, H, 720), (H, I, 721)))
+    else:
+        w13, w2 = _moe_case(fmt, E, 0, H, I, seed=720)
+    moe = MoEWeights(w13.stack(gpu), w2.stack(gpu), H, I, E, 0)
+    rng = np.random.default_rng(T)
+    xb = _x(rng, T, H)
+    rw, rids = O.route(rng.standard_normal((T, E)).astype(np.float32), E)
+    args = (moe, to_dev_bf16(xb, gpu), torch.from_numpy(rw).to(gpu), torch.from_numpy(rids).to(gpu))
+    out, forced = (ops.moe_forward(*args, out_dtype=torch.float32, path=p) for p in (0, 1))
+    ref = O.moe_layer(xb, rids, rw, w13.deq_f32, w2.deq_f32)
+    assert rel_maxabs(out.cpu().numpy(), ref) <= TOL
+    assert rel_maxabs(forced.cpu().numpy(), ref) <= TOL
+    assert not torch.equal(out, forced)
