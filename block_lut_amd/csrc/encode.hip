@@ -214,25 +214,29 @@ __global__ __launch_bounds__(256) void bl4_encode_kernel(const float* __restrict
 //
 // Comparing a weight with every entry costs 3 VALU ops per entry and weight
 // (2816 x 2048 weights, 256 entries: 142 us, 0.12 TB/s, VALU-bound).  Here a
-// CTA sorts the entries once (LDS) and a weight looks up, by its bucket of
-// 1024 over the entries' range, how many entries lie in lower buckets, then
-// steps to its neighbours in the sorted order: about 6 LDS reads and 45 VALU
-// ops a weight (18.4 us for the same weights).  The result is the scan's, bit for bit: rounding is
-// monotone, so the entries at the least rounded distance are a run of the
-// sorted order around v; the run is walked and its lowest index taken.  A run
-// (or an outlier-stretched bucket) only costs time.
+// CTA sorts the entries once (LDS), equal ones kept once, and a weight reads by
+// its bucket of 1024 over the entries' range which sorted values lie in that
+// bucket, searches those (none to two of a trained codebook's) and steps to its
+// neighbours: about 6 LDS reads and 45 VALU ops a weight (19 us for
+// the same weights).  The result is the scan's, bit for bit: rounding is monotone, so the
+// entries at the least rounded distance are a run of the sorted order around v;
+// the run is walked and its lowest index taken.  Where runs can be long
+// (codebooks whose spacing is lost in the distances' rounding) the CTA scans
+// (187 us).  Equal entries walked as runs, and a crowded bucket searched one
+// value after another, took 300 to 940 us (a tier's table, padded with its last
+// entry: 495, now 20).
 enum EncodeRule { kEncode = 0, kQuantizer = 1, kMidpoints = 2 };
 
 constexpr int kEncThreads = 512;
 constexpr int kEncBuckets = 1024;
 
 struct EncTable {
+    float raw[256];                  // entry values, NaN past the last
     float v[258];                    // [0] NaN, then the non-NaN values ascending, then NaN
-    uint8_t idx[256];                // entry of each (equal values in entry order)
-    uint8_t first[kEncBuckets];      // sorted values in lower buckets
-    float lo, scale;
-    int n;                           // non-NaN values
-    float raw[256];
+    uint8_t idx[256];                // entry of each (the lowest of equal ones)
+    uint32_t bucket[kEncBuckets];    // sorted values in lower buckets, and << 16 those in this one
+    uint16_t rank[256];
+    int wsum[4], crowded[4];
 };
 
 // Bucket of v: monotone in v (each step is, with NaN products taken as 0).
@@ -240,57 +244,78 @@ __device__ __forceinline__ int enc_bucket(float v, float lo, float scale) {
     return (int)fminf(fmaxf((v - lo) * scale, 0.f), (float)(kEncBuckets - 1));
 }
 
-// Sorts the m values of s.raw (every thread of the CTA calls it).
-__device__ void enc_build(EncTable& s, int m) {
-    const int t = threadIdx.x;
-    const bool have = t < m && s.raw[t] == s.raw[t];
-    // ascending without NaN (as trained codebooks are): each value is in place
-    const int in_place = __syncthreads_and(t >= m || (have && (t == 0 || s.raw[t - 1] <= s.raw[t])));
-    const int n = __syncthreads_count(have);
-    if (t < 258) s.v[t] = __builtin_nanf("");
-    __syncthreads();
-    if (have) {
-        const float c = s.raw[t];
-        int r = t;
-        if (!in_place) {
-            r = 0;
-            for (int j = 0; j < m; ++j) {
-                const float u = s.raw[j];
-                r += (u < c) || (u == c && j < t);
-            }
-        }
-        s.v[r + 1] = c;
-        s.idx[r] = (uint8_t)t;
-    }
-    __syncthreads();
-    if (t == 0) {
-        const float lo = n ? s.v[1] : 0.f, d = n ? s.v[n] - lo : 0.f;
-        const bool ok = d > 0.f && d < INFINITY;   // (an infinite end: one bucket)
-        s.lo = ok ? lo : 0.f;
-        s.scale = ok ? (float)kEncBuckets / d : 0.f;
-        s.n = n;
-    }
-    __syncthreads();
-    for (int b = t; b < kEncBuckets; b += kEncThreads) {
-        int pos = 0;
+// The entries sorted by value, equal ones once if `once`; returns their number
+// (every thread of the CTA calls it, s.raw complete).  ascending: they are so,
+// without NaN.
+__device__ int enc_sort(EncTable& s, bool ascending, bool once) {
+    static_assert(kEncThreads == 512, "two threads an entry");
+    const int t = threadIdx.x, e = t & 255;
+    const float c = s.raw[e];
+    int r = 0;
+    if (ascending) {
+        r = t < 256 ? e : 0;
+    } else {
+        // rank of entry e, each thread counting one half of the entries: of the
+        // ones before it those up to its value, of the ones after it those below
+        const int e0 = __builtin_amdgcn_readfirstlane(e & ~63);   // the wave's first entry
+        const int j0 = __builtin_amdgcn_readfirstlane(t & 256 ? 128 : 0), j1 = j0 + 128;
+        auto count = [&](int a, int b, auto less) __attribute__((always_inline)) {
+#pragma unroll 1
+            for (int j = max(a, j0); j < min(b, j1); j += 8) {
+                const f32x4_t u = *reinterpret_cast<const f32x4_t*>(&s.raw[j]);
+                const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&s.raw[j + 4]);
 #pragma unroll
-        for (int step = 128; step >= 1; step >>= 1)
-            if (pos + step <= n && enc_bucket(s.v[pos + step], s.lo, s.scale) < b) pos += step;
-        s.first[b] = (uint8_t)pos;   // at most n - 1 for a bucket some v falls in
+                for (int i = 0; i < 8; ++i) r += less(i < 4 ? u[i & 3] : w[i & 3], j + i);
+            }
+        };
+        count(0, e0, [&](float u, int) { return u <= c; });
+        count(e0, e0 + 64, [&](float u, int j) { return (u < c) | ((u == c) & (j < e)); });
+        count(e0 + 64, 256, [&](float u, int) { return u < c; });
+    }
+    if (t >= 256) s.rank[e] = (uint16_t)r;
+    if (t < 258) s.v[t] = __builtin_nanf("");
+    int n = __syncthreads_count(t < 256 && c == c);
+    if (t < 256 && c == c) {
+        r += s.rank[e];
+        s.v[r + 1] = c;
+        s.idx[r] = (uint8_t)e;
     }
     __syncthreads();
+    if (once) {
+        const float val = t < 256 ? s.v[t + 1] : 0.f;
+        const uint8_t id = s.idx[e];
+        const bool keep = t < n && (t == 0 || s.v[t] != val);
+        const int kept = __syncthreads_count(keep);
+        const uint64_t b = __ballot(keep);
+        if ((t & 63) == 0 && t < 256) s.wsum[t >> 6] = __popcll(b);
+        __syncthreads();
+        int p = __popcll(b & ((1ull << (t & 63)) - 1ull));
+        for (int w = 0; w < (e >> 6); ++w) p += s.wsum[w];
+        if (keep) {
+            s.v[p + 1] = val;
+            s.idx[p] = id;
+        }
+        if (t >= kept && t < n) s.v[t + 1] = __builtin_nanf("");
+        n = kept;
+        __syncthreads();
+    }
+    return n;
 }
 
 // Code of the normalised weight x.
 template <int kRule>
 __device__ __forceinline__ uint32_t enc_code(const EncTable& s, float x, float lo, float scale, int last, bool none) {
     if (x != x) return kRule == kMidpoints ? (uint32_t)last : 0u;
-    int pos = s.first[enc_bucket(x, lo, scale)];
-    if constexpr (kRule == kMidpoints) {
-        while (s.v[pos + 1] < x) ++pos;
-        return (uint32_t)pos;
+    const uint32_t bk = s.bucket[enc_bucket(x, lo, scale)];
+    int pos = (int)(bk & 0xffffu), left = (int)(bk >> 16);   // of the bucket's values, those below x
+    while (left > 0) {
+        const int half = (left + 1) >> 1;
+        const float u = s.v[pos + half];
+        const bool below = kRule == kMidpoints ? u < x : u <= x;
+        pos = below ? pos + half : pos;
+        left = below ? left - half : half - 1;
     }
-    while (s.v[pos + 1] <= x) ++pos;
+    if constexpr (kRule == kMidpoints) return (uint32_t)pos;
     // neighbours: sorted value pos - 1 <= x < value pos (NaN: there is none)
     const float dl = x - s.v[pos], du = s.v[pos + 1] - x;
     const float d = fminf(dl, du);
@@ -309,6 +334,21 @@ __device__ __forceinline__ uint32_t enc_code(const EncTable& s, float x, float l
     return best;
 }
 
+// The scan: the first of the m entries at the least distance from x.
+__device__ __forceinline__ uint32_t enc_scan(const EncTable& s, float x, int m) {
+    float bd = fabsf(x - s.raw[0]);
+    uint32_t best = 0;
+#pragma unroll 8
+    for (int c = 1; c < m; ++c) {
+        const float dd = fabsf(x - s.raw[c]);
+        if (dd < bd) {
+            bd = dd;
+            best = (uint32_t)c;
+        }
+    }
+    return best;
+}
+
 // kVec: blocks of 8 * 2^i <= 512 weights, 8 weights (16-byte loads) a lane;
 // else any block size, one wave per block.
 template <int kRule, bool kBf16In, bool kVec>
@@ -317,24 +357,71 @@ __global__ __launch_bounds__(kEncThreads) void ref_encode_kernel(const void* __r
                                                                  int block_size, int64_t nblocks,
                                                                  uint8_t* __restrict__ codes,
                                                                  uint16_t* __restrict__ absmax) {
-    __shared__ EncTable s;
+    __shared__ __attribute__((aligned(16))) EncTable s;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    // values searched: the entries, or the midpoints between them
-    const int m = kRule == kMidpoints ? ncb - 1 : ncb;
-    if (t < m) s.raw[t] = kRule == kMidpoints ? (cb[t] + cb[t + 1]) * 0.5f : cb[t];   // (halving is exact)
+    // values searched: the entries, or the midpoints between them (a midpoint
+    // counts as often as it is there; halving is exact)
+    constexpr bool once = kRule != kMidpoints;
+    const int m = once ? ncb : ncb - 1;
+    auto value = [&](int i) __attribute__((always_inline)) { return once ? cb[i] : (cb[i] + cb[i + 1]) * 0.5f; };
+    const float mine = t < m ? value(t) : __builtin_nanf("");
+    const float prev = t > 0 && t < m ? value(t - 1) : -INFINITY;
+    // strictly ascending without NaN (as trained codebooks are): each value is in place
+    if (t < 256) {
+        s.raw[t] = mine;
+        s.v[t + 1] = mine;
+        s.idx[t] = (uint8_t)t;
+        const uint64_t up = __ballot(t >= m || prev <= mine);
+        const uint64_t strict = __ballot(t == 0 || t >= m || prev < mine);
+        if (lane == 0) s.wsum[wv] = (~up == 0) + 2 * (~strict == 0);
+    } else if (t < 258) {
+        s.v[257 * (t - 256)] = __builtin_nanf("");
+    }
     __syncthreads();
-    enc_build(s, m);
-    const float lo = s.lo, scale = s.scale;
-    const bool none = kRule != kMidpoints && (s.n == 0 || s.raw[0] != s.raw[0]);   // entry 0 NaN: nothing is nearer
+    const int order = s.wsum[0] & s.wsum[1] & s.wsum[2] & s.wsum[3];
+    const bool in_place = order == 3 || (!once && order == 1);
+    if (!in_place) __syncthreads();   // (wsum is used again)
+    const int nv = in_place ? m : enc_sort(s, order & 1, once);
+    const float v1 = nv ? s.v[1] : 0.f, d = nv ? s.v[nv] - v1 : 0.f;
+    const bool spread = d > 0.f && d < INFINITY;   // (equal values or an infinite end: one bucket)
+    const float lo = spread ? v1 : 0.f, scale = spread ? (float)kEncBuckets / d : 0.f;
+    const bool none = kRule != kMidpoints && (nv == 0 || s.raw[0] != s.raw[0]);   // entry 0 NaN: nothing is nearer
+    {   // buckets 2 t and 2 t + 1: values below them and below the next one
+        int pos[3] = {0, 0, 0};
+#pragma unroll
+        for (int step = 128; step >= 1; step >>= 1)
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                if (pos[i] + step <= nv && enc_bucket(s.v[pos[i] + step], lo, scale) < 2 * t + i) pos[i] += step;
+        // past the last bucket with values: all (the search stops at 255)
+        if (!spread) {
+            pos[0] = t ? nv : 0;
+            pos[1] = nv;
+        }
+        if (!spread || t == kEncThreads - 1) pos[2] = nv;
+        *reinterpret_cast<u32x2_t*>(&s.bucket[2 * t]) =
+            u32x2_t{(uint32_t)(pos[0] | (pos[1] - pos[0]) << 16), (uint32_t)(pos[1] | (pos[2] - pos[1]) << 16)};
+    }
+    // |x| <= 1, so equal rounded distances are at most 2^-23 (1 + |v|) apart.  Where
+    // nine values lie (twice) that close, whole runs of them can be equally far
+    if (t < 256) {
+        const float u = s.v[t + 1];
+        const uint64_t c = __ballot(t + 8 < nv && s.v[t + 9] - u <= 0x1p-22f * (1.0f + fabsf(u)));
+        if (lane == 0) s.crowded[wv] = c != 0;
+    }
+    __syncthreads();
+    const bool scan = once && (s.crowded[0] | s.crowded[1] | s.crowded[2] | s.crowded[3]);
     // the clamp's bound in the dtype the reference clamps in
     const float floor_v = kRule == kMidpoints ? 1e-12f
                           : kRule == kQuantizer && kBf16In ? bf16_to_f32(f32_to_bf16(1e-10f)) : 1e-10f;
-    auto code_of = [&](float wx, float mx) __attribute__((always_inline)) {
-        float x = wx / mx;
-        if (kRule == kQuantizer && kBf16In) x = bf16_to_f32(f32_to_bf16(x));
-        return enc_code<kRule>(s, x, lo, scale, ncb - 1, none);
+    auto norm = [&](float wx, float mx) __attribute__((always_inline)) {
+        const float x = wx / mx;
+        return kRule == kQuantizer && kBf16In ? bf16_to_f32(f32_to_bf16(x)) : x;
     };
-    if constexpr (kVec) {
+    auto code_of = [&](float wx, float mx) __attribute__((always_inline)) {
+        return enc_code<kRule>(s, norm(wx, mx), lo, scale, ncb - 1, none);
+    };
+    if (kVec && !scan) {
         const int lpb = block_size >> 3;   // lanes per block
         for (int64_t i0 = ((int64_t)blockIdx.x * kEncThreads + t) * 8; i0 - 8 * lane < n;
              i0 += (int64_t)gridDim.x * kEncThreads * 8) {
@@ -387,7 +474,11 @@ __global__ __launch_bounds__(kEncThreads) void ref_encode_kernel(const void* __r
             float mx = 0.f;
             for (int i = lane; i < len; i += 64) mx = fmaxf(mx, fabsf(load(start + i)));
             mx = fmaxf(wave_reduce_max(mx), floor_v);
-            for (int i = lane; i < len; i += 64) codes[start + i] = (uint8_t)code_of(load(start + i), mx);
+            if (scan) {
+                for (int i = lane; i < len; i += 64) codes[start + i] = (uint8_t)enc_scan(s, norm(load(start + i), mx), m);
+            } else {
+                for (int i = lane; i < len; i += 64) codes[start + i] = (uint8_t)code_of(load(start + i), mx);
+            }
             if (lane == 0) absmax[b] = (uint16_t)f32_to_bf16(mx);
         }
     }

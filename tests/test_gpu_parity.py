@@ -1117,6 +1117,14 @@ def _encode_codebook(kind, rng):
         cb[[3, 200]] = [1e6, -1e6]
     elif kind == "constant":
         cb[:] = 0.5
+    elif kind == "tiny":           # every distance rounds to |v|: one tie of all entries
+        cb = (cb * np.float32(1e-20)).astype(np.float32)
+    elif kind == "padded":         # a tier's table: 16 ascending values, the last one repeated
+        cb = np.sort(cb)
+        cb[16:] = cb[15]
+    elif kind == "padded_mixed":   # equal entries apart, out of order, among NaN
+        cb = cb[rng.integers(0, 17, 256)]
+        cb[[4, 99, 255]] = np.nan
     elif kind == "special":        # signed zeros, infinities, NaN
         cb[[0, 9, 17, 30, 31]] = [np.inf, -np.inf, np.nan, 0.0, -0.0]
     elif kind == "first_nan":
@@ -1124,7 +1132,8 @@ def _encode_codebook(kind, rng):
     return cb
 
 
-@pytest.mark.parametrize("kind", ["repeated", "close", "outlier", "constant", "special", "first_nan"])
+@pytest.mark.parametrize("kind", ["repeated", "close", "outlier", "constant", "special", "first_nan", "tiny",
+                                  "padded", "padded_mixed"])
 @pytest.mark.parametrize("n,block_size,offset", [(8 * 4099, 8, 0), (512 * 9 + 13, 512, 0), (5000, 128, 3), (4100, 24, 0)])
 def test_ref_encode_equals_scan(gpu, kind, n, block_size, offset):
     """The encoder's sorted search against the scan it stands for (the first entry at the
@@ -1206,6 +1215,26 @@ def test_ref_quantize_rules_bitexact(gpu, n, block_size, k, bf16):
     i2, b2 = O.ref_encode_midpoints(w, cb, block_size)
     assert np.array_equal(c2.cpu().numpy(), i2)
     assert np.array_equal(a2.view(torch.int16).cpu().numpy().view(np.uint16), b2)
+
+
+@pytest.mark.parametrize("k,distinct", [(256, 16), (256, 64), (40, 7), (2, 1)])
+@pytest.mark.parametrize("block_size", [128, 100])
+def test_ref_quantize_rules_padded_codebook(gpu, k, distinct, block_size):
+    """A tier's table (its first entries, padded with the last one) under both rules: the first
+    of equal entries, and every midpoint below the value counted."""
+    import torch
+    from block_lut_amd.quantizer import quantize
+    rng = np.random.default_rng(k + distinct)
+    cb = O.bf16_to_f32(O.f32_to_bf16(np.sort(rng.uniform(-1, 1, k).astype(np.float32))))
+    cb[distinct:] = cb[distinct - 1]
+    w = rng.standard_normal(3000).astype(np.float32) * 0.02
+    wt = torch.from_numpy(w).to(gpu)
+    c1, _ = quantize(wt, to_dev_bf16(O.f32_to_bf16(cb), gpu), block_size)
+    i1, _ = O.ref_quantize(w, O.f32_to_bf16(cb), block_size, input_is_bf16=False)
+    assert np.array_equal(c1.cpu().numpy(), i1)
+    c2, _ = quantize(wt, torch.from_numpy(cb).to(gpu), block_size, rule="midpoints")
+    i2, _ = O.ref_encode_midpoints(w, cb, block_size)
+    assert np.array_equal(c2.cpu().numpy(), i2)
 
 
 def test_lut_quantizer_train_quantize_decompress(gpu, tmp_path):
