@@ -230,8 +230,12 @@ __global__ __launch_bounds__(64 * kSkWaves) void dense_skinny_kernel(const uint1
 // k-substep ahead of their MFMAs, the next step's first ones right after the
 // barrier that lands its stage.
 //
-// Tiles run row block by row block, each eighth of them on one XCD (a CTA's
-// index modulo 8), so that the token blocks of a weight row share its L2.
+// Each eighth of the tiles runs on one XCD (a CTA's index modulo 8), row block by
+// row block over a group of token blocks: the 32 tiles on its CUs at a time are
+// about as many rows of weights as of tokens, which share its L2.  (All 16 or 32
+// token blocks of a row block at once read a long batch's activations again for
+// every two row blocks, or every one; against that H = 2048, Is = 5632, T = 4096 /
+// 8192 360 / 781 -> 348 / 675 us, H = 4096 697 / 1489 -> 676 / 1305.)
 //
 // A tile's rate is set by how many CUs have one and by the bytes it pulls (a
 // CU streams about 40 GB/s from HBM), so few tokens take small tiles and the
@@ -267,7 +271,7 @@ template <bool kGateUp, int NMW>
 __global__ __launch_bounds__(256, 1) void dense_tile_kernel(const uint16_t* __restrict__ W,
                                                             const uint16_t* __restrict__ src, int T, int H, int I,
                                                             const float* __restrict__ tokw, void* __restrict__ dst,
-                                                            int nxb, int64_t split_stride, TokenWeights tw) {
+                                                            int nxb, int group, int64_t split_stride, TokenWeights tw) {
     using D = DTile<NMW>;
     constexpr int S = D::kStages, L = D::kLoads, kBM = D::kBM;
     __shared__ __attribute__((aligned(16))) uint8_t ring[S * D::kStage];
@@ -283,7 +287,13 @@ __global__ __launch_bounds__(256, 1) void dense_tile_kernel(const uint16_t* __re
     }
     const int tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (tile >= nxb * nyb) return;
-    const int bx = tile / nyb, m0 = (tile - bx * nyb) * kBM;
+    int y0 = 0, gy = nyb, in = tile;   // the group's first token block, their number, the tile in it
+    if (NMW == 4 && group < nyb) {
+        y0 = tile / (group * nxb) * group;
+        gy = min(group, nyb - y0);
+        in -= y0 * nxb;
+    }
+    const int bx = in / gy, m0 = (y0 + in - bx * gy) * kBM;
     const int nk = K / kDBK, kb0 = nk * (int)blockIdx.z / (int)gridDim.z;
     const int nkb = nk * ((int)blockIdx.z + 1) / (int)gridDim.z - kb0;
     const int n0 = bx * (kGateUp ? kDBN / 2 : kDBN);
@@ -493,12 +503,13 @@ int dense_mfma_launch(const uint16_t* W, const uint16_t* src, int T, int H, int 
     }
     const int nxb = dense_row_blocks(kGateUp, H, I);
     const int64_t stride = (int64_t)T * H;
-#define LUTMOE_DENSE_TILE(NMW)                                                                                      \
-    hipLaunchKernelGGL((dense_tile_kernel<kGateUp, NMW>),                                                           \
-                       dim3(8 * ((nxb * ((T + 64 * NMW - 1) / (64 * NMW)) + 7) / 8 + (kGateUp ? (T + 127) / 128 : 0)), \
-                            1, tiles.ns), dim3(256), 0,                                                             \
-                       s, W,                                                                                        \
-                       src, T, H, I, tokw, dst, nxb, stride, tw)
+    // groups of at least 4 blocks of 256 tokens and less than 8 (the smaller tiles have
+    // few blocks; finding the group costs a launch 0.15 us)
+    const int nyb = (T + 64 * tiles.nmw - 1) / (64 * tiles.nmw), ng = nyb < 8 ? 1 : nyb / 4, group = (nyb + ng - 1) / ng;
+    const dim3 grid(8 * ((nxb * nyb + 7) / 8 + (kGateUp ? (T + 127) / 128 : 0)), 1, tiles.ns);
+#define LUTMOE_DENSE_TILE(NMW)                                                                                       \
+    hipLaunchKernelGGL((dense_tile_kernel<kGateUp, NMW>), grid, dim3(256), 0, s, W, src, T, H, I, tokw, dst, nxb,    \
+                       group, stride, tw)
     switch (tiles.nmw) {
         case 1: LUTMOE_DENSE_TILE(1); break;
         case 2: LUTMOE_DENSE_TILE(2); break;

@@ -1737,10 +1737,11 @@ def test_moe_layer_dense_shared_expert(gpu, T, path, gated, logits):
 
 @pytest.mark.parametrize("T,H,Is", [(4, 128, 64), (5, 128, 64), (16, 192, 640), (17, 128, 576), (32, 64, 128),
                                     (33, 192, 64), (64, 128, 2112), (65, 192, 2048), (129, 128, 1088),
-                                    (1024, 64, 1536), (1025, 192, 192)])
+                                    (1024, 64, 1536), (1025, 192, 192), (2049, 192, 1088), (2049, 2176, 64),
+                                    (2900, 192, 1088)])
 def test_dense_shared_expert_shapes(gpu, T, H, Is):
     """The dense shared expert's kernels at their edges (4 / 64 tokens, tiles of 64, 128 and
-    256 tokens and 128 weight rows, K steps left over by the waves or the ring's stages, the
+    256 tokens and 128 weight rows, 9 and 12 blocks of 256 tokens in groups, K steps left over by the waves or the ring's stages, the
     down projection split over K), each result against float64 within its fp32 sums and the
     bf16 rounding of the activations between the projections."""
     import torch
