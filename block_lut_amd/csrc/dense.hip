@@ -129,9 +129,14 @@ __global__ __launch_bounds__(256, 2) void dense_gemv_kernel(const uint16_t* __re
 // both operands (a permutation of k common to the two: each 128-byte line of a
 // row is read whole), two 16x16x32 MFMAs per row tile, token tile and step.
 // The waves' partial sums meet in LDS and are added in wave order.  H = 2048,
-// Is = 5632, gate/up + down with the layer's other launches (10-15 us; the
-// 4-token GEMV passes, which read the weights ceil(T / 4) times): T = 5 / 19 / 32
-// 34.6 / 45.1 / 49.6 us (55.3 / 103.6 / 152.3); T = 4 41.0 with the GEMV.
+// Is = 5632, gate/up + down with the layer's other launches (7-10 us; in brackets
+// the 4-token GEMV passes, which read the weights ceil(T / 4) times): T = 5 / 16 /
+// 32 30.5 / 36.7 / 44.9 us (49.9 / 86.2 / 148.4).
+// The line to the GEMV, us with it / here: at two tokens the GEMV is ahead (H = 2048,
+// Is = 5632 22.8 / 25.9, 4096 x 512 12.5 / 17.7); at three and four neither is
+// everywhere (four tokens: 2048 x 5632 33.5 / 30.7, 4096 x 14336 100 / 84, 512 x 256
+// 16.4 / 14.2, but 2048 x 1408 18.4 / 19.1, 4096 x 512 19.4 / 21.9), and they stay
+// with it; at five it would take two passes.
 constexpr int kSkWaves = 8;
 constexpr int kSkUnroll = 4;   // K steps in flight per wave
 
@@ -237,8 +242,8 @@ __global__ __launch_bounds__(64 * kSkWaves) void dense_skinny_kernel(const uint1
 // every two row blocks, or every one; against that H = 2048, Is = 5632, T = 4096 /
 // 8192 360 / 781 -> 348 / 675 us, H = 4096 697 / 1489 -> 676 / 1305.)
 //
-// A tile's rate is set by how many CUs have one and by the bytes it pulls (a
-// CU streams about 40 GB/s from HBM), so few tokens take small tiles and the
+// A tile's rate is set by how many CUs have one and by the bytes it pulls (50 to
+// 60 GB/s a CU with all of them streaming), so few tokens take small tiles and the
 // down projection (H / 128 row blocks, K = Is) is split over K: its partial
 // rows are added by the kernel that writes the layer's output.  T = 333,
 // H = 2048, Is = 5632 (the tile it replaces: 256 x 256, weights loaded per lane,
