@@ -607,7 +607,7 @@ def nested_tiers(a, ops, N, torch, dev, NestedExpert, NestedStack, MoEWeights, g
     nl = 4   # 4 layer copies: about 1.4 GB, past the Infinity Cache
     layers = [MoEWeights(stack(2 * I, H), stack(H, I), H, I, E, 0) for _ in range(nl)]
     out = {"_nested_touched": {}}
-    for T, path, label in ((16, ops.PATH_GEMV, "decode"), (1024, ops.PATH_MFMA, "prefill")):
+    for T, path, label in ((16, ops.PATH_AUTO, "decode"), (1024, ops.PATH_MFMA, "prefill")):
         steps = []
         touched = {2: 0, 3: 0, 4: 0}
         for L in layers:
