@@ -272,7 +272,7 @@ struct DTile {
     static constexpr int kLoads = (kBM + kDBN) / 32;   // DMAs per thread per stage
 };
 
-template <bool kGateUp, int NMW>
+template <bool kGateUp, int NMW, bool kGroups>
 __global__ __launch_bounds__(256, 1) void dense_tile_kernel(const uint16_t* __restrict__ W,
                                                             const uint16_t* __restrict__ src, int T, int H, int I,
                                                             const float* __restrict__ tokw, void* __restrict__ dst,
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, 1) void dense_tile_kernel(const uint16_t* __re
     const int tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
     if (tile >= nxb * nyb) return;
     int y0 = 0, gy = nyb, in = tile;   // the group's first token block, their number, the tile in it
-    if (NMW == 4 && group < nyb) {
+    if constexpr (kGroups) {
         y0 = tile / (group * nxb) * group;
         gy = min(group, nyb - y0);
         in -= y0 * nxb;
@@ -509,16 +509,18 @@ int dense_mfma_launch(const uint16_t* W, const uint16_t* src, int T, int H, int 
     const int nxb = dense_row_blocks(kGateUp, H, I);
     const int64_t stride = (int64_t)T * H;
     // groups of at least 4 blocks of 256 tokens and less than 8 (the smaller tiles have
-    // few blocks; finding the group costs a launch 0.15 us)
-    const int nyb = (T + 64 * tiles.nmw - 1) / (64 * tiles.nmw), ng = nyb < 8 ? 1 : nyb / 4, group = (nyb + ng - 1) / ng;
+    // few blocks; a kernel that finds its group takes 0.15 us longer, 2.5 at 333 tokens)
+    const int nyb = (T + 64 * tiles.nmw - 1) / (64 * tiles.nmw), ng = tiles.nmw < 4 || nyb < 8 ? 1 : nyb / 4;
+    const int group = (nyb + ng - 1) / ng;
     const dim3 grid(8 * ((nxb * nyb + 7) / 8 + (kGateUp ? (T + 127) / 128 : 0)), 1, tiles.ns);
-#define LUTMOE_DENSE_TILE(NMW)                                                                                       \
-    hipLaunchKernelGGL((dense_tile_kernel<kGateUp, NMW>), grid, dim3(256), 0, s, W, src, T, H, I, tokw, dst, nxb,    \
-                       group, stride, tw)
-    switch (tiles.nmw) {
-        case 1: LUTMOE_DENSE_TILE(1); break;
-        case 2: LUTMOE_DENSE_TILE(2); break;
-        default: LUTMOE_DENSE_TILE(4); break;
+#define LUTMOE_DENSE_TILE(NMW, GROUPS)                                                                               \
+    hipLaunchKernelGGL((dense_tile_kernel<kGateUp, NMW, GROUPS>), grid, dim3(256), 0, s, W, src, T, H, I, tokw, dst, \
+                       nxb, group, stride, tw)
+    switch (ng > 1 ? 0 : tiles.nmw) {
+        case 0: LUTMOE_DENSE_TILE(4, true); break;
+        case 1: LUTMOE_DENSE_TILE(1, false); break;
+        case 2: LUTMOE_DENSE_TILE(2, false); break;
+        default: LUTMOE_DENSE_TILE(4, false); break;
     }
 #undef LUTMOE_DENSE_TILE
     return lutmoe_host::check_launch();
