@@ -308,16 +308,19 @@ __device__ __forceinline__ uint32_t enc_code(const EncTable& s, float x, float l
     if (x != x) return kRule == kMidpoints ? (uint32_t)last : 0u;
     const uint32_t bk = s.bucket[enc_bucket(x, lo, scale)];
     int pos = (int)(bk & 0xffffu), left = (int)(bk >> 16);   // of the bucket's values, those below x
+    // neighbours: sorted value pos - 1 <= x < value pos (NaN: there is none)
+    float vl = s.v[pos], vu = s.v[pos + left + 1];
     while (left > 0) {
         const int half = (left + 1) >> 1;
         const float u = s.v[pos + half];
         const bool below = kRule == kMidpoints ? u < x : u <= x;
         pos = below ? pos + half : pos;
         left = below ? left - half : half - 1;
+        vl = below ? u : vl;
+        vu = below ? vu : u;
     }
     if constexpr (kRule == kMidpoints) return (uint32_t)pos;
-    // neighbours: sorted value pos - 1 <= x < value pos (NaN: there is none)
-    const float dl = x - s.v[pos], du = s.v[pos + 1] - x;
+    const float dl = x - vl, du = vu - x;
     const float d = fminf(dl, du);
     if (none || !(d < INFINITY)) return 0u;   // the scan's start value stands
     uint32_t best = 255u;
