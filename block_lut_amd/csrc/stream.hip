@@ -1,11 +1,14 @@
-// Grouped LUT-GEMM for few tokens per expert (3 tokens and more, up to about
-// 24 positions an expert): weights streamed to registers, looked up
+// Grouped LUT-GEMM for few tokens per expert (3 tokens and more; past 32 tokens
+// up to 27 positions an expert): weights streamed to registers, looked up
 // there, and multiplied on MFMA (16 x 16 x 32, gfx950).
 //
 // It stands between the decode GEMV kernels, which look every weight up again
 // for each pass of one to four tokens and spend VALU dot products and cross-lane
 // sums on them, and the prefill ring kernel, whose 256-row tiles through 150 KB
-// of LDS leave one wave a SIMD.  What bounds it is HBM.  A CTA is 8 waves of 16
+// of LDS leave one wave a SIMD.  What bounds it is HBM where an expert is large
+// (Mixtral shape gate/up 5.0 TB/s, the copy rate); at the Qwen shape (3.0-4.4
+// TB/s) the VALU, issuing 46-57 % of a CU's busy time, and a grid of one or two
+// rounds of the chip.  A CTA is 8 waves of 16
 // weight rows (gate/up: 8 gate and 8 up rows, so the SwiGLU pair meets in one
 // wave) and one work item: up to 16 NM positions of one expert.  Two CTAs a CU,
 // 4 waves a SIMD.
@@ -26,7 +29,8 @@
 //     with every 8 columns in the order the lookups leave their weights in.
 // Results leave the accumulators as runs of 4 outputs of one position.
 //
-// Before / here, us a layer (the GEMV kernels up to 32 tokens, the ring above):
+// Before / here, us a layer (the GEMV kernels up to 32 tokens, the ring above;
+// rotating layers, each pair of figures from one card, and cards differ by 5 %):
 // Qwen shape BL4 T = 32 / 64 / 256 145 / 185 / 195 -> 119 / 129 / 155, REF T = 19 / 64
 // 143 / 231 -> 108 / 144, NestedLUT tiers T = 16 / 64 83 / 183 -> 68 / 111; Mixtral
 // shape BL4 T = 16 / 64 576 / 408 -> 299 / 341 (4.7 TB/s at T = 16).
