@@ -110,9 +110,9 @@ MoeLayout moe_layout(const lutmoe_moe_desc* d, int T, int k) {
     L.dact = o;     o = align_up(o + (Is ? (size_t)T * Is * 2 : 0));
     L.dw = o;       o = align_up(o + (Is ? (size_t)T * 4 : 0));
     // ... last, so that its K splits (up to 8, of up to 2048 rows in all) take
-    // what a workspace holds past one of them; a workspace that would pass the
-    // fixed scratch of lutmoe_moe_forward_noalloc only with them stays within
-    // it (so the size still grows with T)
+    // what a workspace holds past one of them.  They take no workspace past the
+    // fixed scratch of lutmoe_moe_forward_noalloc (a size that passes it with one
+    // result has room for one; so the size still grows with T)
     L.dy = o;
     const size_t row = (size_t)d->hidden * 4;
     L.dy_row = Is ? (size_t)T * row : 0;

@@ -271,8 +271,9 @@ size_t lutmoe_moe_workspace_size(const lutmoe_moe_desc* d, int T, int k);
  * x bf16 [T][H]; topk_w fp32 [T][k]; topk_ids int32 [T][k] in [0, E).
  * `force_path` 0 = auto: the grouped LUT-GEMV kernels for the smallest
  * batches, the weight-streaming MFMA kernels while an expert has few
- * positions, the grouped MFMA LUT-GEMM above; 1 = the GEMV kernels (up to 320
- * experts and 512 (token, slot) pairs, else the LUT-GEMM), 2 = the LUT-GEMM. */
+ * positions, the grouped MFMA LUT-GEMM above; 1 = the GEMV kernels
+ * (LUTMOE_EUNSUPPORTED past 320 experts or 512 (token, slot) pairs), 2 = the
+ * LUT-GEMM. */
 int lutmoe_moe_forward(const lutmoe_moe_desc* d, const void* x_dev, const float* topk_w_dev,
                        const int32_t* topk_ids_dev, int T, int k, void* out_dev,
                        int out_dtype, void* workspace_dev, size_t workspace_bytes,
